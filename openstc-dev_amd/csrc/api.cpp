@@ -14,6 +14,7 @@
 #include <fstream>
 #include <map>
 #include <memory>
+#include <set>
 #include <sstream>
 #include <string>
 #include <vector>
@@ -426,6 +427,16 @@ int upload_mech(ostc_solver *s) {
       h.hi[i * 7 + c] = m.hi[i * 7 + c];
       h.lo[i * 7 + c] = m.lo[i * 7 + c];
     }
+    {
+      // the extrapolation below t_low: h / R = h(t_low) + cp(t_low) (T - t_low)
+      const double *c = &m.lo[i * 7];
+      const double t = m.t_low[i], t2 = t * t, t3 = t2 * t, t4 = t3 * t, t5 = t4 * t;
+      h.cp_ext[i] = c[0] + c[1] * t + c[2] * t2 + c[3] * t3 + c[4] * t4;
+      h.h_ext[i] = c[0] * t + 0.5 * c[1] * t2 + c[2] * t3 / 3 + 0.25 * c[3] * t4 + 0.2 * c[4] * t5 + c[5] -
+                   h.cp_ext[i] * t;
+      h.log_t_low[i] = std::log(t);
+      h.t_low_inv[i] = 1 / t;
+    }
     h.LJ_potent_inv[i] = m.LJ_potent_inv[i];
     h.log_LJ_potent_inv[i] = m.LJ_potent_inv[i] > 0 ? std::log(m.LJ_potent_inv[i]) : 0.0;
     h.vis_coeff[i] = m.vis_coeff[i];
@@ -457,6 +468,9 @@ int upload_mech(ostc_solver *s) {
     h.stoi_b[i] = m.stoi_b[i];
     h.third_body_coeff[i] = m.third_body_coeff[i];
   }
+  std::set<double> brk(m.t_low.begin(), m.t_low.begin() + ns);
+  brk.insert(m.t_mid.begin(), m.t_mid.begin() + ns);
+  h.n_brk = (int)(std::copy(brk.begin(), brk.end(), h.brk) - h.brk);
   HIPCHK(hipMalloc(&s->d_mech, sizeof(DMech)));
   HIPCHK(hipMemcpy(s->d_mech, &h, sizeof(DMech), hipMemcpyHostToDevice));
   return 0;

@@ -36,7 +36,7 @@ __device__ inline double d_ipow(double x, int n) {
 // FiniteRateChem.cu:65-149 for reaction r: kf (Arrhenius + duplicate, third
 // body, Lindemann, Troe) and kb = kf / Kc (or the REV set, 0 if irreversible).
 template <int NS>
-__device__ inline void d_rate(const DMech *__restrict__ m, int r, double t, double lt, double it, const double *c,
+__device__ inline void d_rate(MechK m, int r, double t, double lt, double it, const double *c,
                               const double *g, double temp_t, double &kf, double &kb) {
   const int type = m->label[r];
   double k = d_arrhenius(lt, it, m->A[r], m->b[r], m->Ea[r]);
@@ -85,11 +85,11 @@ __device__ inline void d_rate(const DMech *__restrict__ m, int r, double t, doub
 // and source are fused per reaction so no per-reaction array is kept.
 // omega_d (may be null): the destruction rates [kg/m3/s] of chemical_source.
 template <int NS>
-__device__ inline void d_chem_source(const DMech *__restrict__ m, double rho, double t, const double *Y, double *omega,
+__device__ inline void d_chem_source(MechK m, double rho, double t, const double *Y, double *omega,
                                      double *jac, double *omega_d = nullptr) {
   double c[NS], g[NS];
 #pragma unroll
-  for (int l = 0; l < NS; ++l) c[l] = rho * Y[l] / m->mw[l] * 1e-3;
+  for (int l = 0; l < NS; ++l) c[l] = d_div(rho * Y[l], m->mw[l], m->mw_inv[l]) * 1e-3;
   d_gibbs_rt<NS>(t, m, g);
   const double temp_t = (kPatmD() / kRuD * 1e-3) / t;
   const double lt = log(t), it = 1.0 / t;
@@ -154,11 +154,11 @@ __device__ inline void d_chem_source(const DMech *__restrict__ m, double rho, do
 // keeps the kernel in registers.  Sums run over r in the same order as in
 // d_chem_source, so the results are the same.
 template <int NS>
-__device__ inline void d_chem_rates(const DMech *__restrict__ m, double rho, double t, const double *Y, double *omega,
+__device__ inline void d_chem_rates(MechK m, double rho, double t, const double *Y, double *omega,
                                     double *q, int stride) {
   double c[NS], g[NS];
 #pragma unroll
-  for (int l = 0; l < NS; ++l) c[l] = rho * Y[l] / m->mw[l] * 1e-3;
+  for (int l = 0; l < NS; ++l) c[l] = d_div(rho * Y[l], m->mw[l], m->mw_inv[l]) * 1e-3;
   d_gibbs_rt<NS>(t, m, g);
   const double temp_t = (kPatmD() / kRuD * 1e-3) / t;
   const double lt = log(t), it = 1.0 / t;
@@ -195,7 +195,7 @@ __device__ inline void d_chem_rates(const DMech *__restrict__ m, double rho, dou
 
 // The EPI Jacobian J from the parked rates of progress; with EPI, A = I - dt J
 template <int NS, bool EPI = true>
-__device__ inline void d_epi_matrix(const DMech *__restrict__ m, double rho, const double *Y, double dt,
+__device__ inline void d_epi_matrix(MechK m, double rho, const double *Y, double dt,
                                     const double *q, int stride, double *A) {
 #pragma unroll
   for (int a = 0; a < NS * NS; ++a) A[a] = 0;
@@ -291,7 +291,7 @@ __device__ inline void d_lu_solve(double *A, double *b) {
 // with T*^-0.145 = exp(-0.145 (log T + log(kb/eps))); also sqrt(vis) and
 // 1 / sqrt(vis), so that Wilke's sqrt(vis_a / vis_b) is a product
 template <int NS>
-__device__ inline void species_viscosities(const DMech *__restrict__ m, double t, double *vis, double *sv,
+__device__ inline void species_viscosities(MechK m, double t, double *vis, double *sv,
                                            double *isv) {
   const double st = sqrt(t), lt = log(t);
 #pragma unroll
@@ -307,11 +307,11 @@ __device__ inline void species_viscosities(const DMech *__restrict__ m, double t
 // Transport.cu:113-140 compute_viscosity: Wilke's rule alone, at the mean
 // molecular weight mw_total of composition Y
 template <int NS>
-__device__ inline double d_viscosity(const DMech *__restrict__ m, double t, double mw_total, const double *Y) {
+__device__ inline double d_viscosity(MechK m, double t, double mw_total, const double *Y) {
   double X[NS], vis[NS], sv[NS], isv[NS];
   species_viscosities<NS>(m, t, vis, sv, isv);
 #pragma unroll
-  for (int l = 0; l < NS; ++l) X[l] = Y[l] * mw_total / m->mw[l];
+  for (int l = 0; l < NS; ++l) X[l] = Y[l] * mw_total * m->mw_inv[l];
   double mu = 0;
 #pragma unroll
   for (int a = 0; a < NS; ++a) {
@@ -332,17 +332,17 @@ __device__ inline double d_viscosity(const DMech *__restrict__ m, double t, doub
 
 // Transport.cu:40-110 compute_transport_property
 template <int NS>
-__device__ inline void d_transport(const DMech *__restrict__ m, double t, double p, double rho, const double *Y,
+__device__ inline void d_transport(MechK m, double t, double p, double rho, const double *Y,
                                    const double *cp, double &mu, double &lam, double *rhoD) {
   double mwi = 0;
 #pragma unroll
-  for (int l = 0; l < NS; ++l) mwi += Y[l] / m->mw[l];
+  for (int l = 0; l < NS; ++l) mwi += Y[l] * m->mw_inv[l];
   const double mw_total = 1 / mwi;
   double X[NS], vis[NS], sv[NS], isv[NS];
   const double st = sqrt(t);
   species_viscosities<NS>(m, t, vis, sv, isv);
 #pragma unroll
-  for (int l = 0; l < NS; ++l) X[l] = Y[l] * mw_total / m->mw[l];
+  for (int l = 0; l < NS; ++l) X[l] = Y[l] * mw_total * m->mw_inv[l];
   double viscosity = 0, conductivity = 0;
 #pragma unroll
   for (int a = 0; a < NS; ++a) {
@@ -358,7 +358,7 @@ __device__ inline void d_transport(const DMech *__restrict__ m, double t, double
     }
     const double ct = 1.065 * vt - 0.065 * X[a];
     viscosity += vis[a] * X[a] / vt;
-    const double la = vis[a] * (cp[a] + 1.25 * kRuD / m->mw[a]);
+    const double la = vis[a] * (cp[a] + 1.25 * kRuD * m->mw_inv[a]);
     conductivity += la * X[a] / ct;
   }
   mu = viscosity;

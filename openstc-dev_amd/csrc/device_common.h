@@ -18,6 +18,13 @@ constexpr int kMR = 50;   // reaction capacity of the device tables
 struct DMech {
   int n_spec, n_reac;
   double mw[kMS], mw_inv[kMS], t_low[kMS], t_mid[kMS], hi[kMS * 7], lo[kMS * 7];
+  // below t_low: cp / R stays cp(t_low) and h / R = h_ext + cp_ext T
+  double cp_ext[kMS], h_ext[kMS];
+  double log_t_low[kMS], t_low_inv[kMS];
+  // the different t_low and t_mid of all species, ascending: between two of
+  // them every species keeps its branch
+  int n_brk;
+  double brk[2 * kMS];
   double LJ_potent_inv[kMS], vis_coeff[kMS];
   double WjDivWi_to_One4th[kMS * kMS], sqrt_WiDivWjPl1Mul8[kMS * kMS];
   double binary_diffusivity_coeff[kMS * kMS], kb_over_eps_jk[kMS * kMS];
@@ -90,94 +97,172 @@ constexpr double kMwAirD = 28.9647;
 // ---------------------------------------------------------------- thermo
 // Thermo.cu:5-79.  Below t_low: h extrapolated with cp(t_low), cp and g/RT
 // frozen at t_low.
+//
+// The tables are read through a pointer into the constant address space, so
+// every load is a scalar one (uniform address, never aliased by the kernel's
+// stores), and each species takes its temperature branch by selecting the
+// value, not the coefficients: a coefficient pointer chosen per lane made
+// each evaluation 6 or 7 vector loads per species behind divergent branches,
+// some 700 of the 980 vector loads of a 9-species AWENO face.  With the
+// branch-free forms, the mixture polynomial below and products with 1 / W_l
+// in place of quotients: 512x256 mixing layer 2.69 -> 1.71 ms per RK3 step,
+// 192x96x64 channel 12.5 -> 8.6 ms per pseudo-iteration; the 9-species AWENO
+// sweeps no longer use scratch memory.
+typedef const __attribute__((address_space(4))) DMech *MechK;
+__device__ inline MechK mech_k(const DMech *m) { return (MechK)m; }
 
 // The mechanism pointer made opaque to the optimiser: a property evaluation
-// given fresh(m) loads its NASA-7 coefficients where it uses them
-// (scalar-cache hits) instead of sharing loads hoisted once and held in
-// registers for the rest of the kernel (the flux sweeps evaluate the
-// properties at many temperatures per face).
-__device__ inline const DMech *fresh(const DMech *m) {
+// given fresh(m) loads its coefficients where it uses them (scalar-cache
+// hits) instead of sharing loads hoisted once and held in registers for the
+// rest of the kernel (the flux sweeps evaluate the properties at many
+// temperatures per face).
+__device__ inline MechK fresh(MechK m) {
   asm volatile("" : "+s"(m));
   return m;
 }
 
+// a / b for a finite a and a normal quotient, with rb = 1 / b correctly
+// rounded: the residual of a * rb is exact in a fused multiply-add, and adding
+// its share back rounds to the quotient itself (Markstein 1990), so the result
+// is the one a division gives, in 3 operations instead of 11.
+__device__ inline double d_div(double a, double b, double rb) {
+  const double q = a * rb;
+  return fma(fma(-b, q, a), rb, q);
+}
+
+// T and the weights of a0 .. a4 in h / R = a0 T + a1 T^2 / 2 + .. + a4 T^5 / 5 + a5
+struct TPow {
+  double t, t2, t3, t4, p2, p3, p4, p5;
+  __device__ explicit TPow(double T) : t(T) {
+    t2 = t * t;
+    t3 = t2 * t;
+    t4 = t3 * t;
+    p2 = 0.5 * t2;
+    p3 = t3 * (1.0 / 3);
+    p4 = 0.25 * t4;
+    p5 = 0.2 * (t4 * t);
+  }
+};
+
+// h_l of species l at T
+__device__ inline double d_species_h(MechK m, int l, const TPow &q) {
+  const auto *a = &m->lo[l * 7];
+  const auto *b = &m->hi[l * 7];
+  const double hl = fma(a[4], q.p5, fma(a[3], q.p4, fma(a[2], q.p3, fma(a[1], q.p2, fma(a[0], q.t, a[5])))));
+  const double hh = fma(b[4], q.p5, fma(b[3], q.p4, fma(b[2], q.p3, fma(b[1], q.p2, fma(b[0], q.t, b[5])))));
+  const double he = fma(m->cp_ext[l], q.t, m->h_ext[l]);
+  const double h = q.t < m->t_mid[l] ? hl : hh;
+  return (q.t < m->t_low[l] ? he : h) * m->r_mw[l];
+}
+
+// cp_l of species l at T
+__device__ inline double d_species_cp(MechK m, int l, const TPow &q) {
+  const auto *a = &m->lo[l * 7];
+  const auto *b = &m->hi[l * 7];
+  const double cl = fma(a[4], q.t4, fma(a[3], q.t3, fma(a[2], q.t2, fma(a[1], q.t, a[0]))));
+  const double ch = fma(b[4], q.t4, fma(b[3], q.t3, fma(b[2], q.t2, fma(b[1], q.t, b[0]))));
+  const double c = q.t < m->t_mid[l] ? cl : ch;
+  return (q.t < m->t_low[l] ? (double)m->cp_ext[l] : c) * m->r_mw[l];
+}
+
 template <int NS>
-__device__ inline void d_enthalpy(double t, const DMech *__restrict__ m, double *h) {
-  const double t2 = t * t, t3 = t2 * t, t4 = t3 * t, t5 = t4 * t;
+__device__ inline void d_enthalpy(double t, MechK m, double *h) {
+  const TPow q(t);
 #pragma unroll
   for (int i = 0; i < NS; ++i) {
-    if (t < m->t_low[i]) {
-      const double tt = m->t_low[i];
-      const double tt2 = tt * tt, tt3 = tt2 * tt, tt4 = tt3 * tt, tt5 = tt4 * tt;
-      const double *c = &m->lo[i * 7];
-      double hh = c[0] * tt + 0.5 * c[1] * tt2 + c[2] * tt3 / 3 + 0.25 * c[3] * tt4 + 0.2 * c[4] * tt5 + c[5];
-      const double cp = c[0] + c[1] * tt + c[2] * tt2 + c[3] * tt3 + c[4] * tt4;
-      h[i] = hh + cp * (t - tt);
-    } else {
-      const double *c = t < m->t_mid[i] ? &m->lo[i * 7] : &m->hi[i * 7];
-      h[i] = c[0] * t + 0.5 * c[1] * t2 + c[2] * t3 / 3 + 0.25 * c[3] * t4 + 0.2 * c[4] * t5 + c[5];
-    }
-    h[i] *= m->r_mw[i];
+    if (i % 4 == 0) m = fresh(m);
+    h[i] = d_species_h(m, i, q);
   }
 }
 
 template <int NS>
-__device__ inline void d_enthalpy_cp(double t, const DMech *__restrict__ m, double *h, double *cp) {
-  const double t2 = t * t, t3 = t2 * t, t4 = t3 * t, t5 = t4 * t;
+__device__ inline void d_enthalpy_cp(double t, MechK m, double *h, double *cp) {
+  const TPow q(t);
 #pragma unroll
   for (int i = 0; i < NS; ++i) {
-    if (t < m->t_low[i]) {
-      const double tt = m->t_low[i];
-      const double tt2 = tt * tt, tt3 = tt2 * tt, tt4 = tt3 * tt, tt5 = tt4 * tt;
-      const double *c = &m->lo[i * 7];
-      const double hh = c[0] * tt + 0.5 * c[1] * tt2 + c[2] * tt3 / 3 + 0.25 * c[3] * tt4 + 0.2 * c[4] * tt5 + c[5];
-      cp[i] = c[0] + c[1] * tt + c[2] * tt2 + c[3] * tt3 + c[4] * tt4;
-      h[i] = hh + cp[i] * (t - tt);
-    } else {
-      const double *c = t < m->t_mid[i] ? &m->lo[i * 7] : &m->hi[i * 7];
-      h[i] = c[0] * t + 0.5 * c[1] * t2 + c[2] * t3 / 3 + 0.25 * c[3] * t4 + 0.2 * c[4] * t5 + c[5];
-      cp[i] = c[0] + c[1] * t + c[2] * t2 + c[3] * t3 + c[4] * t4;
-    }
-    h[i] *= m->r_mw[i];
-    cp[i] *= m->r_mw[i];
+    if (i % 3 == 0) m = fresh(m);
+    h[i] = d_species_h(m, i, q);
+    cp[i] = d_species_cp(m, i, q);
   }
 }
 
 template <int NS>
-__device__ inline void d_cp(double t, const DMech *__restrict__ m, double *cp) {
-  const double t2 = t * t, t3 = t2 * t, t4 = t3 * t;
+__device__ inline void d_cp(double t, MechK m, double *cp) {
+  const TPow q(t);
 #pragma unroll
   for (int i = 0; i < NS; ++i) {
-    const double tt = t < m->t_low[i] ? m->t_low[i] : t;
-    const double *c = (t < m->t_low[i] || t < m->t_mid[i]) ? &m->lo[i * 7] : &m->hi[i * 7];
-    if (t < m->t_low[i]) {
-      const double tt2 = tt * tt, tt3 = tt2 * tt, tt4 = tt3 * tt;
-      cp[i] = c[0] + c[1] * tt + c[2] * tt2 + c[3] * tt3 + c[4] * tt4;
-    } else {
-      cp[i] = c[0] + c[1] * t + c[2] * t2 + c[3] * t3 + c[4] * t4;
-    }
-    cp[i] *= m->r_mw[i];
+    if (i % 4 == 0) m = fresh(m);
+    cp[i] = d_species_cp(m, i, q);
   }
 }
 
 template <int NS>
-__device__ inline void d_gibbs_rt(double t, const DMech *__restrict__ m, double *g) {
-  const double t2 = t * t, t3 = t2 * t, t4 = t3 * t, t_inv = 1 / t, log_t = log(t);
+__device__ inline void d_gibbs_rt(double t, MechK m, double *g) {
+  const double log_t = log(t), t_inv = 1 / t;
 #pragma unroll
   for (int i = 0; i < NS; ++i) {
-    if (t < m->t_low[i]) {
-      const double tt = m->t_low[i];
-      const double tt2 = tt * tt, tt3 = tt2 * tt, tt4 = tt3 * tt, tt_inv = 1 / tt, log_tt = log(tt);
-      const double *c = &m->lo[i * 7];
-      g[i] = c[0] * (1.0 - log_tt) - 0.5 * c[1] * tt - c[2] * tt2 / 6.0 - c[3] * tt3 / 12.0 - c[4] * tt4 * 0.05 +
-             c[5] * tt_inv - c[6];
-    } else {
-      const double *c = t < m->t_mid[i] ? &m->lo[i * 7] : &m->hi[i * 7];
-      g[i] = c[0] * (1.0 - log_t) - 0.5 * c[1] * t - c[2] * t2 / 6.0 - c[3] * t3 / 12.0 - c[4] * t4 * 0.05 +
-             c[5] * t_inv - c[6];
-    }
+    if (i % 3 == 0) m = fresh(m);
+    // frozen at t_low below it
+    const bool cold = t < m->t_low[i];
+    const double x = cold ? (double)m->t_low[i] : t, x2 = x * x, x3 = x2 * x, x4 = x3 * x;
+    const double lx = cold ? (double)m->log_t_low[i] : log_t, xi = cold ? (double)m->t_low_inv[i] : t_inv;
+    auto poly = [&](double c0, double c1, double c2, double c3, double c4, double c5, double c6) {
+      return c0 * (1.0 - lx) - 0.5 * c1 * x - d_div(c2 * x2, 6.0, 1 / 6.0) - d_div(c3 * x3, 12.0, 1 / 12.0) -
+             c4 * x4 * 0.05 + c5 * xi - c6;
+    };
+    const auto *a = &m->lo[i * 7];
+    const auto *b = &m->hi[i * 7];
+    const double gl = poly(a[0], a[1], a[2], a[3], a[4], a[5], a[6]);
+    const double gh = poly(b[0], b[1], b[2], b[3], b[4], b[5], b[6]);
+    g[i] = cold || x < m->t_mid[i] ? gl : gh;
   }
 }
+
+// sum_l w_l h_l(T) and sum_l w_l cp_l(T) as one polynomial in T, its
+// coefficients the weighted sums of the species': each species adds its own
+// branch at T, so the polynomial is exact on [ta, tb), the interval between
+// two branch points around T.  One construction costs about one evaluation
+// of all species; a Newton iteration then costs ten multiply-adds instead of
+// twenty per species.
+struct MixPoly {
+  double a0, a1, a2, a3, a4, a5, ta, tb;
+
+  // the coefficients are loaded for two species at a time (fresh): loaded all
+  // at once they overflow the scalar registers into vector-register lanes
+  template <int NS>
+  __device__ inline void build(MechK m, const double *w, double t) {
+    a0 = a1 = a2 = a3 = a4 = a5 = 0;
+#pragma unroll
+    for (int l = 0; l < NS; ++l) {
+      if (l % 2 == 0) m = fresh(m);
+      const double x = w[l] * m->r_mw[l];
+      const bool cold = t < m->t_low[l], low = t < m->t_mid[l];
+      const double xl = low && !cold ? x : 0.0, xh = low || cold ? 0.0 : x, xe = cold ? x : 0.0;
+      const auto *a = &m->lo[l * 7];
+      const auto *b = &m->hi[l * 7];
+      a0 = fma(xl, a[0], fma(xh, b[0], fma(xe, m->cp_ext[l], a0)));
+      a1 = fma(xl, a[1], fma(xh, b[1], a1));
+      a2 = fma(xl, a[2], fma(xh, b[2], a2));
+      a3 = fma(xl, a[3], fma(xh, b[3], a3));
+      a4 = fma(xl, a[4], fma(xh, b[4], a4));
+      a5 = fma(xl, a[5], fma(xh, b[5], fma(xe, m->h_ext[l], a5)));
+    }
+    ta = -1e300;
+    tb = 1e300;
+    const int nb = m->n_brk;
+    for (int i = 0; i < nb; ++i) {
+      const double b = m->brk[i];
+      const bool above = t >= b;
+      ta = above ? b : ta;
+      tb = !above && b < tb ? b : tb;
+    }
+  }
+  __device__ inline bool holds(double t) const { return t >= ta && t < tb; }
+  __device__ inline double cp(double t) const { return fma(t, fma(t, fma(t, fma(t, a4, a3), a2), a1), a0); }
+  __device__ inline double h(double t) const {
+    return fma(t, fma(t, fma(t, fma(t, fma(t, 0.2 * a4, 0.25 * a3), (1.0 / 3) * a2), 0.5 * a1), a0), a5);
+  }
+};
 
 // Transport.cu:6-9
 // (T / 273)^1.5 as x sqrt(x): the same power within an ulp, without the
@@ -190,27 +275,21 @@ __device__ inline double d_sutherland(double t) {
 // FieldOperation.cu:3-39: Newton on e(T) from the warm start; tolerance
 // |1 - T1/T| <= 1e-3, at most 1000 iterations.
 template <int NS>
-__device__ inline double d_temperature(const DMech *__restrict__ m, double rho, double rhoE, double u, double v,
-                                       double w, const double *Y, double t, double &p) {
-  double mw = 0;
+__device__ inline double d_temperature(MechK m, double rho, double rhoE, double u, double v, double w, const double *Y,
+                                       double t, double &p) {
+  double mwi = 0;
 #pragma unroll
-  for (int l = 0; l < NS; ++l) mw += Y[l] / m->mw[l];
-  mw = 1 / mw;
-  const double gas = kRuD / mw;
+  for (int l = 0; l < NS; ++l) mwi += Y[l] * m->mw_inv[l];
+  const double gas = kRuD * mwi;
   const double e = rhoE / rho - 0.5 * (u * u + v * v + w * w);
+  MixPoly q;
+  q.ta = q.tb = 0;  // built in the loop
   double err = 1;
   int iter = 0;
   while (err > 1e-3 && iter++ < 1000) {
-    double h[NS > 0 ? NS : 1], cp[NS > 0 ? NS : 1];
-    d_enthalpy_cp<NS>(t, m, h, cp);
-    double cpt = 0, ht = 0;
-#pragma unroll
-    for (int l = 0; l < NS; ++l) {
-      cpt += cp[l] * Y[l];
-      ht += h[l] * Y[l];
-    }
-    const double et = ht - gas * t;
-    const double cv = cpt - gas;
+    if (!q.holds(t)) q.build<NS>(m, Y, t);
+    const double et = q.h(t) - gas * t;
+    const double cv = q.cp(t) - gas;
     const double t1 = t - (et - e) / cv;
     err = fabs(1 - t1 / t);
     t = t1;

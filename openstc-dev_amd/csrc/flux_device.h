@@ -52,7 +52,7 @@ __device__ inline R minmod(R a, R b) {
 // otherwise first order: the two adjacent points only).  Appends rhoE at
 // [nv] and gamma at [nv+1].
 template <int NS, int NT, typename R>
-__device__ inline void recon_pv(const ZoneView &z, int recon, const DMech *__restrict__ m, int64_t p0, int64_t st,
+__device__ inline void recon_pv(const ZoneView &z, int recon, MechK m, int64_t p0, int64_t st,
                                 R *pl, R *pr) {
   constexpr int NV = 5 + NS + NT;
   const R kappa = R(1.0 / 3.0);
@@ -82,26 +82,22 @@ __device__ inline void recon_pv(const ZoneView &z, int recon, const DMech *__res
     double mil = 0, mir = 0;
 #pragma unroll
     for (int l = 0; l < NS; ++l) {
-      mil += (double)pl[5 + l] / m->mw[l];
-      mir += (double)pr[5 + l] / m->mw[l];
+      mil += (double)pl[5 + l] * m->mw_inv[l];
+      mir += (double)pr[5 + l] * m->mw_inv[l];
     }
     const double tl = (double)pl[4] / ((double)pl[0] * kRuD * mil), tr = (double)pr[4] / ((double)pr[0] * kRuD * mir);
-    double h[NS], c[NS];
-    double cpl = 0, cvl = 0, cpr = 0, cvr = 0;
-    d_enthalpy_cp<NS>(tl, fresh(m), h, c);
+    double y[NS];
+    MixPoly q;
 #pragma unroll
-    for (int l = 0; l < NS; ++l) {
-      cpl += c[l] * (double)pl[l + 5];
-      cvl += (double)pl[l + 5] * (c[l] - m->r_mw[l]);
-      el += h[l] * (double)pl[l + 5];
-    }
-    d_enthalpy_cp<NS>(tr, fresh(m), h, c);
+    for (int l = 0; l < NS; ++l) y[l] = (double)pl[5 + l];
+    q.build<NS>(m, y, tl);
+    el += q.h(tl);
+    const double cpl = q.cp(tl), cvl = cpl - kRuD * mil;
 #pragma unroll
-    for (int l = 0; l < NS; ++l) {
-      cpr += c[l] * (double)pr[l + 5];
-      cvr += (double)pr[l + 5] * (c[l] - m->r_mw[l]);
-      er += h[l] * (double)pr[l + 5];
-    }
+    for (int l = 0; l < NS; ++l) y[l] = (double)pr[5 + l];
+    q.build<NS>(m, y, tr);
+    er += q.h(tr);
+    const double cpr = q.cp(tr), cvr = cpr - kRuD * mir;
     pl[NV] = (R)((double)pl[0] * el - (double)pl[4]);
     pr[NV] = (R)((double)pr[0] * er - (double)pr[4]);
     pl[NV + 1] = (R)(cpl / cvl);
@@ -327,7 +323,7 @@ struct MixEig {
 // Roe state of the face between cl and cr = (Q[NV], p); k0/k1 the metric
 // rows of the sweep direction at the two points
 template <int NS, int NT, typename R>
-__device__ inline void mix_roe_state(const DMech *__restrict__ m, const R *cl, const R *cr, const R *k0, const R *k1,
+__device__ inline void mix_roe_state(MechK m, const R *cl, const R *cr, const R *k0, const R *k1,
                                      MixEig<NS, NT, R> &E) {
   constexpr int NV = 5 + NS + NT;
   const R dl = sqrt(cl[0]), dr = sqrt(cr[0]), id = rcp(dl + dr);
@@ -343,17 +339,20 @@ __device__ inline void mix_roe_state(const DMech *__restrict__ m, const R *cl, c
   if constexpr (NS > 0) {
     double mwi = 0;
 #pragma unroll
-    for (int l = 0; l < NS; ++l) mwi += (double)E.y[l] / m->mw[l];
+    for (int l = 0; l < NS; ++l) mwi += (double)E.y[l] * m->mw_inv[l];
     const double t = (double)((dl * (cl[NV] * il) + dr * (cr[NV] * ir)) * id) / (kRuD * mwi);
-    double hi[NS], cpi[NS];
-    d_enthalpy_cp<NS>(t, fresh(m), hi, cpi);
-    double cp = 0, cv = 0, hs = 0;
+    double hi[NS];
+    double cp = 0, hs = 0;
+    const TPow tp(t);
+    MechK mk = m;
 #pragma unroll
     for (int l = 0; l < NS; ++l) {
-      cp += cpi[l] * (double)E.y[l];
-      cv += (double)E.y[l] * (cpi[l] - m->r_mw[l]);
+      if (l % 3 == 0) mk = fresh(mk);
+      hi[l] = d_species_h(mk, l, tp);
+      cp += d_species_cp(mk, l, tp) * (double)E.y[l];
       hs += (double)E.y[l] * hi[l];
     }
+    const double cv = cp - kRuD * mwi;
     const double gamma = cp / cv;
     const double c = sqrt(gamma * kRuD * mwi * t);
     const double mw = 1 / mwi;
@@ -364,8 +363,8 @@ __device__ inline void mix_roe_state(const DMech *__restrict__ m, const R *cl, c
     const double c2 = c * c, g2 = (gamma - 1) / c2, cg = c2 / (gamma - 1);
 #pragma unroll
     for (int l = 0; l < NS; ++l) {
-      E.a[l] = (R)(mw / m->mw[l] - hi[l] * g2);
-      E.b[l] = (R)(hi[l] - mw / m->mw[l] * cg);
+      E.a[l] = (R)(mw * m->mw_inv[l] - hi[l] * g2);
+      E.b[l] = (R)(hi[l] - mw * m->mw_inv[l] * cg);
     }
   } else {
     E.t = 0;
@@ -426,36 +425,33 @@ __device__ inline void mix_right(const MixEig<NS, NT, R> &E, const R *wv, R *Q) 
 
 // Temperature of a mixture of mass fractions Y at internal energy e per unit
 // mass: Newton on sum Y h(T) - R T sum Y/W = e from t0, until |dT| <= 1e-12 T
-// (at most 30 iterations).  FP64 in every precision mode.
+// (at most 30 iterations); also sum Y/W and the mixture's cp there.  FP64 in
+// every precision mode.
 template <int NS>
-__device__ inline double d_energy_temperature(const DMech *__restrict__ m, const double *Y, double e, double t0,
-                                              double &mwi) {
+__device__ inline double d_energy_temperature(MechK m, const double *Y, double e, double t0, double &mwi, double &cp) {
   mwi = 0;
 #pragma unroll
-  for (int l = 0; l < NS; ++l) mwi += Y[l] / m->mw[l];
+  for (int l = 0; l < NS; ++l) mwi += Y[l] * m->mw_inv[l];
+  const double gas = kRuD * mwi;
   double t = t0;
-  for (int it = 0; it < 30; ++it) {
-    double h[NS], cp[NS];
-    d_enthalpy_cp<NS>(t, fresh(m), h, cp);
-    double f = 0, fp = 0;
-#pragma unroll
-    for (int l = 0; l < NS; ++l) {
-      f += Y[l] * h[l];
-      fp += Y[l] * cp[l];
-    }
-    f -= kRuD * t * mwi + e;
-    fp -= kRuD * mwi;
-    const double dt = f / fp;
+  MixPoly q;
+  q.ta = q.tb = 0;
+  bool last = false;
+  for (int it = 0;; ++it) {
+    if (!q.holds(t)) q.build<NS>(m, Y, t);
+    if (last) break;
+    const double dt = (q.h(t) - gas * t - e) / (q.cp(t) - gas);
     t -= dt;
-    if (fabs(dt) <= 1e-12 * t) break;
+    last = fabs(dt) <= 1e-12 * t || it == 29;
   }
+  cp = q.cp(t);
   return t;
 }
 
 // primitives (rho, u, v, w, p, scalars; rho E at [NV], gamma at [NV+1]) of a
 // reconstructed conservative side Q
 template <int NS, int NT, typename R>
-__device__ inline void mix_side(const DMech *__restrict__ m, const MixEig<NS, NT, R> &E, const R *Q, R *pv) {
+__device__ inline void mix_side(MechK m, const MixEig<NS, NT, R> &E, const R *Q, R *pv) {
   constexpr int NV = 5 + NS + NT;
   const R rho = Q[0], ri = rcp(rho);
   pv[0] = rho;
@@ -467,19 +463,12 @@ __device__ inline void mix_side(const DMech *__restrict__ m, const MixEig<NS, NT
   const R ek = R(0.5) * (pv[1] * pv[1] + pv[2] * pv[2] + pv[3] * pv[3]);
   pv[NV] = Q[4];
   if constexpr (NS > 0) {
-    double Y[NS], mwi;
+    double Y[NS], mwi, cp;
 #pragma unroll
     for (int l = 0; l < NS; ++l) Y[l] = (double)pv[5 + l];
-    const double t = d_energy_temperature<NS>(m, Y, (double)(Q[4] * ri - ek), E.t, mwi);
+    const double t = d_energy_temperature<NS>(m, Y, (double)(Q[4] * ri - ek), E.t, mwi, cp);
     pv[4] = (R)((double)rho * kRuD * t * mwi);
-    double cpi[NS];
-    d_cp<NS>(t, fresh(m), cpi);
-    double cp = 0, cv = 0;
-#pragma unroll
-    for (int l = 0; l < NS; ++l) {
-      cp += cpi[l] * Y[l];
-      cv += Y[l] * (cpi[l] - m->r_mw[l]);
-    }
+    const double cv = cp - kRuD * mwi;
     pv[NV + 1] = (R)(cp / cv);
   } else {
     pv[4] = R(kGam - 1) * (Q[4] - ek * rho);
@@ -514,7 +503,7 @@ __device__ inline bool mix_side_ok(const R *pv) {
 // 6 x NV amplitude block of the whole stencil is never live at once; the
 // arithmetic and its order are those of mix_left / weno5 per component.
 template <int NS, int NT, typename R>
-__device__ inline void aweno_mix(const ZoneView &z, const DMech *__restrict__ m, int64_t p0, int64_t st,
+__device__ inline void aweno_mix(const ZoneView &z, MechK m, int64_t p0, int64_t st,
                                  const R *mk0, const R *mk1, R *pl, R *pr) {
   constexpr int NV = 5 + NS + NT;
   MixEig<NS, NT, R> E;
@@ -660,7 +649,7 @@ __device__ inline void face_vector(const R *mk0, const R *mk1, R j0, R j1, bool 
 
 // HLLC.cu:10-143
 template <int NS, int NT, typename R>
-__device__ inline void hllc(const DMech *__restrict__ m, const R *pl, const R *pr, const R *mk0, const R *mk1, R j0,
+__device__ inline void hllc(MechK m, const R *pl, const R *pr, const R *mk0, const R *mk1, R j0,
                             R j1, bool jface, R *f) {
   constexpr int NV = 5 + NS + NT;
   const R sl0 = sqrt(pl[0]), sr0 = sqrt(pr[0]);
@@ -679,16 +668,18 @@ __device__ inline void hllc(const DMech *__restrict__ m, const R *pl, const R *p
 #pragma unroll
     for (int l = 0; l < NS; ++l) {
       svm[l] = (double)(rlc * pl[l + 5] + rrc * pr[l + 5]);
-      mwi += svm[l] / m->mw[l];
+      mwi += svm[l] * m->mw_inv[l];
     }
     const double t = (double)(rlc * (pl[4] * ipl) + rrc * (pr[4] * ipr)) / (kRuD * mwi);
-    double h[NS], c[NS], cpp = 0, cvv = 0;
-    d_enthalpy_cp<NS>(t, fresh(m), h, c);
+    double cpp = 0;
+    const TPow tp(t);
+    MechK mk = m;
 #pragma unroll
     for (int l = 0; l < NS; ++l) {
-      cpp += c[l] * svm[l];
-      cvv += svm[l] * (c[l] - m->r_mw[l]);
+      if (l % 4 == 0) mk = fresh(mk);
+      cpp += d_species_cp(mk, l, tp) * svm[l];
     }
+    const double cvv = cpp - kRuD * mwi;
     ct = (R)sqrt(cpp / cvv * kRuD * mwi * t);
   }
   R kx, ky, kz, ja;
@@ -777,7 +768,7 @@ __device__ inline R efix_point(const ZoneView &z, const DParams &P, int64_t p) {
 // Roe-averaged temperature, FP64), Harten's entropy fix with the face
 // average of the point deltas d0, d1.
 template <int NS, int NT, typename R>
-__device__ inline void roe(const DMech *__restrict__ m, const R *pl, const R *pr, const R *mk0, const R *mk1, R j0,
+__device__ inline void roe(MechK m, const R *pl, const R *pr, const R *mk0, const R *mk1, R j0,
                            R j1, R d0, R d1, R *f) {
   constexpr int NV = 5 + NS + NT;
 #pragma unroll
@@ -811,10 +802,10 @@ __device__ inline void roe(const DMech *__restrict__ m, const R *pl, const R *pr
   } else {
     double mwi = 0;
 #pragma unroll
-    for (int l = 0; l < NS; ++l) mwi += (double)svm[l] / m->mw[l];
+    for (int l = 0; l < NS; ++l) mwi += (double)svm[l] * m->mw_inv[l];
     const double t = (double)((dl * (pl[4] / pl[0]) + dr * (pr[4] / pr[0])) * id) / (kRuD * mwi);
     double hh[NS], cc[NS], cp = 0, cv = 0;
-    d_enthalpy_cp<NS>(t, fresh(m), hh, cc);
+    d_enthalpy_cp<NS>(t, m, hh, cc);
 #pragma unroll
     for (int l = 0; l < NS; ++l) {
       cp += cc[l] * (double)svm[l];
@@ -849,7 +840,7 @@ __device__ inline void roe(const DMech *__restrict__ m, const R *pl, const R *pr
   R c1 = g1 * (ek * dq[0] - u * dq[1] - v * dq[2] - w * dq[3] + dq[4]) * ic2;
   R c2 = (kx * dq[1] + ky * dq[2] + kz * dq[3] - Uk * dq[0]) / c;
 #pragma unroll
-  for (int l = 0; l < NS; ++l) c1 += (mw / (R)m->mw[l] - hi[l] * g1 * ic2) * dq[l + 5];
+  for (int l = 0; l < NS; ++l) c1 += (mw * (R)m->mw_inv[l] - hi[l] * g1 * ic2) * dq[l + 5];
   R c3 = dq[0] - c1;
   R b[NV];
   b[0] = -lam[0] * (R(0.5) * (c1 - c2));
@@ -864,7 +855,7 @@ __device__ inline void roe(const DMech *__restrict__ m, const R *pl, const R *pr
   c2 = c * (b[4] - b[0]);
   c3 = R(0);
 #pragma unroll
-  for (int l = 0; l < NS; ++l) c3 += (hi[l] - mw / (R)m->mw[l] * c * c / g1) * b[l + 5];
+  for (int l = 0; l < NS; ++l) c3 += (hi[l] - mw * (R)m->mw_inv[l] * c * c / g1) * b[l + 5];
   f[0] += R(0.5) * c1;
   f[1] += R(0.5) * (u * c1 + kx * c2 - c * (kz * b[2] - ky * b[3]));
   f[2] += R(0.5) * (v * c1 + ky * c2 - c * (kx * b[3] - kz * b[1]));
@@ -903,7 +894,7 @@ __device__ inline void lax_friedrichs(const R *pl, const R *pr, const R *mk0, co
 // stress, Fourier flux, mixture-averaged diffusion with the correction
 // velocity; the flux is projected on the J-weighted face metric.
 template <int NS, int NT, typename R>
-__device__ inline void viscous_face(const ZoneView &z, const DParams &P, const DMech *__restrict__ m, int dir,
+__device__ inline void viscous_face(const ZoneView &z, const DParams &P, MechK m, int dir,
                                     int64_t p0, int64_t st, R *fv) {
   const int64_t p1 = p0 + st;
   const int64_t so[3] = {1, z.d2, z.d1};
@@ -985,8 +976,8 @@ __device__ inline void viscous_face(const ZoneView &z, const DParams &P, const D
       const R gg = kx * yx[0] + ky * yx[1] + kz * yx[2];
       ddf[l] = gg;
       corr += dif[l] * gg;
-      sum_gy_w += gg / (R)m->mw[l];
-      mw_tot += yk[l] / (R)m->mw[l];
+      sum_gy_w += gg * (R)m->mw_inv[l];
+      mw_tot += yk[l] * (R)m->mw_inv[l];
       sum_rdy += dif[l] * yk[l];
     }
     mw_tot = R(1.0) / mw_tot;
@@ -999,17 +990,18 @@ __device__ inline void viscous_face(const ZoneView &z, const DParams &P, const D
                     (R(0.5) * ((R)z.bv[4 * z.sz + p1] + (R)z.bv[4 * z.sz + p0]));
 #pragma unroll
       for (int l = 0; l < NS; ++l) {
-        ddf[l] += (mw_tot / (R)m->mw[l] - R(1)) * yk[l] * gpp;
-        corr += (mw_tot / (R)m->mw[l] - R(1)) * yk[l] * gpp * dif[l];
+        ddf[l] += (mw_tot * (R)m->mw_inv[l] - R(1)) * yk[l] * gpp;
+        corr += (mw_tot * (R)m->mw_inv[l] - R(1)) * yk[l] * gpp * dif[l];
       }
     }
-    double h[NS];
-    d_enthalpy<NS>(0.5 * (z.bv[5 * z.sz + p0] + z.bv[5 * z.sz + p1]), fresh(m), h);
+    const TPow tp(0.5 * (z.bv[5 * z.sz + p0] + z.bv[5 * z.sz + p1]));
+    MechK mk = m;
 #pragma unroll
     for (int l = 0; l < NS; ++l) {
+      if (l % 4 == 0) mk = fresh(mk);
       const R df = dif[l] * (ddf[l] - mw_tot * yk[l] * sum_gy_w) - yk[l] * corr;
       fv[5 + l] = df;
-      fv[4] += (R)h[l] * df;
+      fv[4] += (R)d_species_h(mk, l, tp) * df;
     }
   }
   if constexpr (NT > 0) {
@@ -1082,7 +1074,7 @@ __device__ inline R cds_weight(int s) {
 // Riemann solver on the reconstructed states plus the viscous flux:
 // F(face) = inviscid - viscous.
 template <int NS, int NT, int SCHEME, typename R>
-__device__ inline void riemann_viscous(const ZoneView &z, const DParams &P, const DMech *__restrict__ m, int dir,
+__device__ inline void riemann_viscous(const ZoneView &z, const DParams &P, MechK m, int dir,
                                        int64_t p0, int64_t st, const R *pl, const R *pr, const R *mk0, const R *mk1,
                                        R j0, R j1, R *F) {
   constexpr int NV = 5 + NS + NT;
@@ -1112,7 +1104,7 @@ __device__ inline void riemann_viscous(const ZoneView &z, const DParams &P, cons
 // (several kernels use it) its arrays and the kernel arguments went to the
 // stack.
 template <int NS, int NT, int SCHEME, typename R>
-__device__ __attribute__((always_inline)) inline void face_flux(const ZoneView &z, const DParams &P, const DMech *__restrict__ m, int dir, int64_t p0,
+__device__ __attribute__((always_inline)) inline void face_flux(const ZoneView &z, const DParams &P, MechK m, int dir, int64_t p0,
                                  int64_t st, bool want_g, R *F, R *G) {
   constexpr int NV = 5 + NS + NT;
   constexpr int NG = CdsWidth<NS, NT, SCHEME>::value;
@@ -1186,7 +1178,8 @@ __device__ inline int xcd_logical_block(int hw, int nb) {
 // the end of a row; lane l's cell takes its left face from lane l - 1
 // through a cross-lane shuffle.
 template <int NS, int NT, int SCHEME, typename R>
-__global__ void __launch_bounds__(256) sweep_i(ZoneView z, DParams P, const DMech *__restrict__ m, int init, int bpp) {
+__global__ void __launch_bounds__(256) sweep_i(ZoneView z, DParams P, const DMech *__restrict__ mech, int init, int bpp) {
+  const MechK m = mech_k(mech);
   constexpr int NV = 5 + NS + NT;
   const int lane = threadIdx.x;
   const int n = z.mx;
@@ -1224,8 +1217,9 @@ __global__ void __launch_bounds__(256) sweep_i(ZoneView z, DParams P, const DMec
 constexpr int kISlots = 288;
 
 template <typename R>
-__global__ void __launch_bounds__(256) sweep_i_aweno(ZoneView z, DParams P, const DMech *__restrict__ m, int init,
+__global__ void __launch_bounds__(256) sweep_i_aweno(ZoneView z, DParams P, const DMech *__restrict__ mech, int init,
                                                      int bpp) {
+  const MechK m = mech_k(mech);
   __shared__ R sQ[6][kISlots];  // cv 0..4, p
   __shared__ R sN[5][kISlots];  // node flux
   const int lane = threadIdx.x, tid = threadIdx.y * 64 + lane;
@@ -1329,8 +1323,9 @@ __device__ inline JkLine jk_line(const ZoneView &z, int gx, int nseg) {
 
 template <int DIR, int NS, int NT, int SCHEME, typename R>
 __global__ void __launch_bounds__((64 * JkRows<NS + NT, R>::value)) sweep_jk(ZoneView z, DParams P,
-                                                                           const DMech *__restrict__ m, int init,
+                                                                           const DMech *__restrict__ mech, int init,
                                                                            int gx, int nseg) {
+  const MechK m = mech_k(mech);
   constexpr int NV = 5 + NS + NT;
   constexpr int NG = CdsWidth<NS, NT, SCHEME>::value;  // the CDS flux G exists for AWENO only
   constexpr int kRows = JkRows<NS + NT, R>::value;
@@ -1388,8 +1383,9 @@ __global__ void __launch_bounds__((64 * JkRows<NS + NT, R>::value)) sweep_jk(Zon
 // over its cells in dt_partial[blockIdx.x] -- the stand-alone time-step pass
 // folded into the last sweep of the right-hand side.
 template <int DIR, int kRows, typename R, bool DT = false>
-__global__ void __launch_bounds__(64 * kRows) sweep_jk_aweno(ZoneView z, DParams P, const DMech *__restrict__ m,
+__global__ void __launch_bounds__(64 * kRows) sweep_jk_aweno(ZoneView z, DParams P, const DMech *__restrict__ mech,
                                                              int init, int gx, int nseg, double *dt_partial) {
+  const MechK m = mech_k(mech);
   constexpr int kRing = kRows + 5;
   __shared__ R sQ[kRing][6][64];     // cv 0..4, p
   __shared__ R sN[kRing][5][64];     // node flux

@@ -94,7 +94,7 @@ __global__ void __launch_bounds__(kTB) k_dplur_dq0(ZoneView z, int fr, int chem,
 
 // DPLUR.cuh:80-137: (A +- lambda I) dq at point (i, j, k) along dir
 template <int NS, int NT>
-__device__ inline void jac_times_dq(const ZoneView &z, const DMech *__restrict__ m, int i, int j, int k, int dir,
+__device__ inline void jac_times_dq(const ZoneView &z, MechK m, int i, int j, int k, int dir,
                                     double lam, double *out) {
   constexpr int NV = 5 + NS + NT;
   const int64_t p = z.at(i, j, k), q = z.at0(i, j, k);
@@ -117,7 +117,7 @@ __device__ inline void jac_times_dq(const ZoneView &z, const DMech *__restrict__
     gamma = z.gam[p];
 #pragma unroll
     for (int l = 0; l < NS; ++l) {
-      b3 += kRuD * t / m->mw[l] * d[5 + l];
+      b3 += kRuD * t * m->mw_inv[l] * d[5 + l];
       b4 += z.dplur_h[(int64_t)l * z.sz0 + q] * d[5 + l];
     }
     h = z.dplur_h[(int64_t)NS * z.sz0 + q];
@@ -139,7 +139,8 @@ __device__ inline void jac_times_dq(const ZoneView &z, const DMech *__restrict__
 // at the point's temperature and h = sum_l Y_l h_l + |u|^2 / 2, summed in the
 // order the Jacobian product uses
 template <int NS>
-__global__ void __launch_bounds__(kTB) k_dplur_enthalpy(ZoneView z, const DMech *__restrict__ m) {
+__global__ void __launch_bounds__(kTB) k_dplur_enthalpy(ZoneView z, const DMech *__restrict__ mech) {
+  const MechK m = mech_k(mech);
   int i, j, k;
   if (!cell_index(z, i, j, k)) return;
   const int64_t p = z.at(i, j, k), q = z.at0(i, j, k);
@@ -195,7 +196,7 @@ __device__ inline void dplur_finish(const ZoneView &z, int i, int j, int k, cons
 
 // the i- and j-neighbour term of one side: tot += s 0.5 (A +- lambda I) dq
 template <int NS, int NT>
-__device__ inline void dplur_add(const ZoneView &z, const DMech *__restrict__ m, int i, int j, int k, int dir,
+__device__ inline void dplur_add(const ZoneView &z, MechK m, int i, int j, int k, int dir,
                                  double sign, double *tot) {
   constexpr int NV = 5 + NS + NT;
   double jd[NV];
@@ -212,8 +213,9 @@ __device__ inline void dplur_add(const ZoneView &z, const DMech *__restrict__ m,
 // DPLUR.cuh:139-257: dqk from the neighbours' current dq (interior only), one
 // thread per cell
 template <int NS, int NT>
-__global__ void __launch_bounds__(kTB) k_dplur_inner(ZoneView z, const DMech *__restrict__ m, int fr, int chem,
+__global__ void __launch_bounds__(kTB) k_dplur_inner(ZoneView z, const DMech *__restrict__ mech, int fr, int chem,
                                                      int timp) {
+  const MechK m = mech_k(mech);
   constexpr int NV = 5 + NS + NT;
   int i, j, k;
   if (!cell_index(z, i, j, k)) return;
@@ -259,7 +261,8 @@ __global__ void k_dq_back(ZoneView z, const double *__restrict__ src, int nv) {
 // scalars advanced by dq dt_local / J from the old primitives; then T and p
 // (Newton from the energy for mixtures).  cv is not touched.
 template <int NS>
-__global__ void __launch_bounds__(kTB) k_update_bv(ZoneView z, DParams P, const DMech *__restrict__ m) {
+__global__ void __launch_bounds__(kTB) k_update_bv(ZoneView z, DParams P, const DMech *__restrict__ mech) {
+  const MechK m = mech_k(mech);
   int i, j, k;
   if (!cell_index(z, i, j, k)) return;
   const int64_t p = z.at(i, j, k), q = z.at0(i, j, k);

@@ -83,7 +83,8 @@ __device__ inline double sst_mut(const ZoneView &z, int ns, int64_t p, double mu
 
 // FieldOperation.cuh:175-195 initialize_mut on [-1, m]
 template <int NS>
-__global__ void __launch_bounds__(kTB) k_init_mut(ZoneView z, const DMech *__restrict__ m) {
+__global__ void __launch_bounds__(kTB) k_init_mut(ZoneView z, const DMech *__restrict__ mech) {
+  const MechK m = mech_k(mech);
   const int X = z.mx + 2, Y = z.my + 2, Z = z.mz + 2;
   const int64_t t = (int64_t)blockIdx.x * kTB + threadIdx.x;
   if (t >= (int64_t)X * Y * Z) return;
@@ -100,7 +101,7 @@ __global__ void __launch_bounds__(kTB) k_init_mut(ZoneView z, const DMech *__res
 #pragma unroll
     for (int l = 0; l < NS; ++l) {
       Yk[l] = z.sv[(int64_t)l * z.sz + p];
-      mwi += Yk[l] / m->mw[l];
+      mwi += Yk[l] * m->mw_inv[l];
     }
     mul = d_viscosity<NS>(m, T, 1 / mwi, Yk);
   }

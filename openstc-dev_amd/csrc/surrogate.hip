@@ -49,10 +49,10 @@ struct SurNorm {
 
 // (log(Y + 1e-12), T, log p) of one cell; p from the equation of state as
 // in the point-implicit batch kernel
-__device__ inline void raw_features(const DMech *__restrict__ m, double rho, double T, const double *Y, double *x) {
+__device__ inline void raw_features(MechK m, double rho, double T, const double *Y, double *x) {
   double mwi = 0;
 #pragma unroll
-  for (int l = 0; l < kNS; ++l) mwi += Y[l] / m->mw[l];
+  for (int l = 0; l < kNS; ++l) mwi += Y[l] * m->mw_inv[l];
   const double mw = 1 / mwi;
   const double p = rho * T * (kRuD / mw);
 #pragma unroll
@@ -68,10 +68,11 @@ __device__ inline void load_cell(int64_t n, int64_t c, const double *__restrict_
 
 // raw features F [n x 16] and raw targets Tt [n x 16]: null-space coordinates
 // of dY, dT and sigma_min(I - dt J)
-__global__ void k_sur_raw(const DMech *__restrict__ m, int64_t n, const double *__restrict__ rho,
+__global__ void k_sur_raw(const DMech *__restrict__ mech, int64_t n, const double *__restrict__ rho,
                           const double *__restrict__ T, const double *__restrict__ Y_a, const double *__restrict__ dY,
                           const double *__restrict__ dT, const double *__restrict__ sig, SurNorm nm,
                           float *__restrict__ F, float *__restrict__ Tt) {
+  const MechK m = mech_k(mech);
   const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (c >= n) return;
   double Y[kNS], x[kSurIn], d[kNS];
@@ -163,9 +164,10 @@ __global__ void k_pack_x(int64_t B, const float *__restrict__ x, __bf16 *__restr
 }
 
 // standardised network inputs of cells c0 .. c0+count
-__global__ void k_sur_features(const DMech *__restrict__ m, int64_t n, int64_t c0, int64_t count,
+__global__ void k_sur_features(const DMech *__restrict__ mech, int64_t n, int64_t c0, int64_t count,
                                const double *__restrict__ rho, const double *__restrict__ T,
                                const double *__restrict__ Y_a, SurNorm nm, __bf16 *__restrict__ X) {
+  const MechK m = mech_k(mech);
   const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (t >= count) return;
   const int64_t c = c0 + t;
@@ -195,7 +197,7 @@ __global__ void k_sur_features(const DMech *__restrict__ m, int64_t n, int64_t c
 // 2 non-finite output, 3 |dY_k| above dy_max, 4 |dT| above dT_max,
 // 5 sigma_min below sig_min, 6 conservation error above cons_tol,
 // 7 temperature inversion failed.
-__device__ inline int finish_cell(const DMech *__restrict__ m, const SurNorm &nm, int64_t n, int64_t c,
+__device__ inline int finish_cell(MechK m, const SurNorm &nm, int64_t n, int64_t c,
                                    const double *__restrict__ rho_a, const double *__restrict__ T_a,
                                    const double *__restrict__ Y_a, const float *o, double *__restrict__ dY,
                                    double *__restrict__ dT) {
@@ -209,7 +211,7 @@ __device__ inline int finish_cell(const DMech *__restrict__ m, const SurNorm &nm
     // Y + 1e-12, T and p against the exponentiated bounds
     double mwi = 0;
 #pragma unroll
-    for (int l = 0; l < kNS; ++l) mwi += Y[l] / m->mw[l];
+    for (int l = 0; l < kNS; ++l) mwi += Y[l] * m->mw_inv[l];
     const double p = rho * T * (kRuD / (1 / mwi));
 #pragma unroll
     for (int l = 0; l < kNS; ++l) {
@@ -259,7 +261,7 @@ __device__ inline int finish_cell(const DMech *__restrict__ m, const SurNorm &nm
   if (ok) {
     double mwi = 0, h[kNS];
 #pragma unroll
-    for (int l = 0; l < kNS; ++l) mwi += Y[l] / m->mw[l];
+    for (int l = 0; l < kNS; ++l) mwi += Y[l] * m->mw_inv[l];
     const double mw = 1 / mwi;
     const double p_old = rho * T * (kRuD / mw);
     d_enthalpy<kNS>(T, m, h);
@@ -309,13 +311,14 @@ __device__ inline void append_fallback(bool fb, int64_t c, int *__restrict__ fb_
   if (fb) fb_idx[base + (int)__popcll(mask & ((1ull << lane) - 1ull))] = (int)c;
 }
 
-__global__ void __launch_bounds__(256) k_sur_finish(const DMech *__restrict__ m, SurNorm nm, int64_t n, int64_t c0,
+__global__ void __launch_bounds__(256) k_sur_finish(const DMech *__restrict__ mech, SurNorm nm, int64_t n, int64_t c0,
                                                     int64_t count, const double *__restrict__ rho_a,
                                                     const double *__restrict__ T_a, const double *__restrict__ Y_a,
                                                     const float *__restrict__ out, int ld, int force_fallback,
                                                     double *__restrict__ dY, double *__restrict__ dT,
                                                     int *__restrict__ fb_count, int *__restrict__ fb_idx,
                                                     int *__restrict__ reasons) {
+  const MechK m = mech_k(mech);
   __shared__ int s_codes[9];
   __shared__ int s_wave[4];
   __shared__ int s_base;
@@ -345,11 +348,12 @@ __global__ void __launch_bounds__(256) k_sur_finish(const DMech *__restrict__ m,
 // FP32.  Writes the standardised outputs out[c * 8 + j]; the gate runs in
 // k_sur_finish.  LDS: R x 264 BF16 (66 kB for R = 128), two workgroups per CU.
 template <int R, int PF>
-__global__ void __launch_bounds__(256, 2) k_sur_net(const DMech *__restrict__ m, SurNorm nm, int64_t n,
+__global__ void __launch_bounds__(256, 2) k_sur_net(const DMech *__restrict__ mech, SurNorm nm, int64_t n,
                                                     int64_t count, const double *__restrict__ rho_a,
                                                     const double *__restrict__ T_a, const double *__restrict__ Y_a,
                                                     const __bf16 *__restrict__ wb, int64_t off1, int64_t off2,
                                                     int64_t off3, float *__restrict__ out) {
+  const MechK m = mech_k(mech);
   static_assert(R % 64 == 0 && R <= 256, "rows per workgroup");
   constexpr int RT = R / 16;
   __shared__ __bf16 act[R][kHld];
@@ -489,12 +493,13 @@ __global__ void __launch_bounds__(256, 2) k_sur_net(const DMech *__restrict__ m,
 // (Ml(h): layer-l products of half h, El(h): its epilogue, O: output layer).
 // Every product and epilogue is the one of k_sur_net, in the same order.
 template <int PF>
-__global__ void __launch_bounds__(256, 2) k_sur_net_pipe(const DMech *__restrict__ m, SurNorm nm, int64_t n,
+__global__ void __launch_bounds__(256, 2) k_sur_net_pipe(const DMech *__restrict__ mech, SurNorm nm, int64_t n,
                                                          int64_t count, const double *__restrict__ rho_a,
                                                          const double *__restrict__ T_a,
                                                          const double *__restrict__ Y_a,
                                                          const __bf16 *__restrict__ wb, int64_t off1, int64_t off2,
                                                          int64_t off3, float *__restrict__ out) {
+  const MechK m = mech_k(mech);
   constexpr int R = 128, RT = 8;
   __shared__ __bf16 act[R][kHld];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;

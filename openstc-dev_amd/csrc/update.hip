@@ -44,7 +44,8 @@ constexpr int kSrcTB = 128;
 constexpr int kParkMaxReac = 24;  // reactions per cell the LDS park holds
 
 template <int NS>
-__global__ void __launch_bounds__(kSrcTB) k_source(ZoneView z, DParams P, const DMech *__restrict__ m, int accumulate) {
+__global__ void __launch_bounds__(kSrcTB) k_source(ZoneView z, DParams P, const DMech *__restrict__ mech, int accumulate) {
+  const MechK m = mech_k(mech);
   extern __shared__ double sq_park[];
   const int64_t t = (int64_t)blockIdx.x * kSrcTB + threadIdx.x;
   const int64_t n = (int64_t)z.mx * z.my * z.mz;
@@ -131,8 +132,9 @@ __global__ void __launch_bounds__(kTB) k_min_final(const double *partial, int nb
 // ------------------------------------------------------------- RK update
 // RK.cuh:10-14 (SSP-RK3 a, b, c) and RK.cuh:197-253 update_cv_and_bv_rk.
 template <int NS>
-__global__ void __launch_bounds__(kTB) k_rk_update(ZoneView z, DParams P, const DMech *__restrict__ m,
+__global__ void __launch_bounds__(kTB) k_rk_update(ZoneView z, DParams P, const DMech *__restrict__ mech,
                                                     const double *__restrict__ dtp, int rk) {
+  const MechK m = mech_k(mech);
   const int64_t t = (int64_t)blockIdx.x * kTB + threadIdx.x;
   const int64_t n = (int64_t)z.mx * z.my * z.mz;
   if (t >= n) return;
@@ -196,7 +198,7 @@ __global__ void __launch_bounds__(kTB) k_rk_update(ZoneView z, DParams P, const 
 
 // FieldOperation.cuh:18-110 compute_total_energy / compute_cv_from_bv_1_point
 template <int NS>
-__device__ inline void cv_point(const ZoneView &z, const DMech *__restrict__ m, int64_t p, int nt) {
+__device__ inline void cv_point(const ZoneView &z, MechK m, int64_t p, int nt) {
   const double rho = z.bv[p], u = z.bv[z.sz + p], v = z.bv[2 * z.sz + p], w = z.bv[3 * z.sz + p];
   for (int l = NS; l < NS + nt; ++l) z.cv[(int64_t)(5 + l) * z.sz + p] = rho * z.sv[(int64_t)l * z.sz + p];
   z.cv[p] = rho;
@@ -225,7 +227,8 @@ __device__ inline void cv_point(const ZoneView &z, const DMech *__restrict__ m, 
 }
 
 template <int NS>
-__global__ void __launch_bounds__(kTB) k_cv_from_bv(ZoneView z, const DMech *__restrict__ m, int nt) {
+__global__ void __launch_bounds__(kTB) k_cv_from_bv(ZoneView z, const DMech *__restrict__ mech, int nt) {
+  const MechK m = mech_k(mech);
   const int X = z.mx + 2 * z.g, Y = z.my + 2 * z.g, Z = z.mz + 2 * z.g;
   const int64_t t = (int64_t)blockIdx.x * kTB + threadIdx.x;
   if (t >= (int64_t)X * Y * Z) return;
@@ -247,8 +250,9 @@ __global__ void __launch_bounds__(kTB) k_velocity(ZoneView z) {
 // take the target's interior values.  Threads touch disjoint points: the
 // ghost layers read target points off its face layer.
 template <int NS, bool WITH_CV>
-__global__ void __launch_bounds__(kTB) k_inner_exchange(ZoneView z, ZoneView tz, const DMech *__restrict__ m,
+__global__ void __launch_bounds__(kTB) k_inner_exchange(ZoneView z, ZoneView tz, const DMech *__restrict__ mech,
                                                         InnerFaceDesc f, int nsc, int nt) {
+  const MechK m = mech_k(mech);
   const int64_t t = (int64_t)blockIdx.x * kTB + threadIdx.x;
   const int64_t n01 = (int64_t)f.n[0] * f.n[1];
   if (t >= n01 * f.n[2]) return;
@@ -296,7 +300,8 @@ __global__ void __launch_bounds__(kTB) k_inner_exchange(ZoneView z, ZoneView tz,
 // Lanes run along the face's fastest index: the layer for i-faces (ghosts
 // adjacent in memory), the point for j- and k-faces.
 template <int NS, bool WITH_CV>
-__global__ void __launch_bounds__(kTB) k_bc(ZoneView z, DParams P, const DMech *__restrict__ m, BCDesc b) {
+__global__ void __launch_bounds__(kTB) k_bc(ZoneView z, DParams P, const DMech *__restrict__ mech, BCDesc b) {
+  const MechK m = mech_k(mech);
   const int nx = b.re[0] - b.rs[0] + 1, ny = b.re[1] - b.rs[1] + 1, nz = b.re[2] - b.rs[2] + 1;
   const uint32_t npt = (uint32_t)nx * ny * nz, nl = z.g + 1;
   const uint32_t t = blockIdx.x * kTB + threadIdx.x;
@@ -404,7 +409,7 @@ __global__ void __launch_bounds__(kTB) k_bc(ZoneView z, DParams P, const DMech *
 #pragma unroll
       for (int l = 0; l < NS; ++l) {
         svb[l] = sv[l * S + p];
-        mi += svb[l] / m->mw[l];
+        mi += svb[l] * m->mw_inv[l];
       }
       gb = z.gam[p];
       mw = 1 / mi;
@@ -570,7 +575,7 @@ __global__ void __launch_bounds__(kTB) k_bc(ZoneView z, DParams P, const DMech *
 #pragma unroll
       for (int l = 0; l < NS; ++l) {
         Yw[l] = sv[l * S + pi];
-        s += Yw[l] / m->mw[l];
+        s += Yw[l] * m->mw_inv[l];
       }
       mw = 1 / s;
     }
@@ -617,7 +622,7 @@ __global__ void __launch_bounds__(kTB) k_bc(ZoneView z, DParams P, const DMech *
         for (int l = 0; l < NS; ++l) {
           const double y = sv[l * S + pa];
           sv[l * S + pg] = y;
-          s += y / m->mw[l];
+          s += y * m->mw_inv[l];
         }
         mw = 1 / s;
       }
@@ -674,7 +679,8 @@ __global__ void __launch_bounds__(kTB) k_eliminate_k(ZoneView z, DParams P) {
 // stored on k = -1, 0, 1 (bit-identical to computing each plane), the Mach
 // number from each plane's own |u|.
 template <int NS, bool PLANE>
-__global__ void __launch_bounds__(kTB) k_properties(ZoneView z, DParams P, const DMech *__restrict__ m) {
+__global__ void __launch_bounds__(kTB) k_properties(ZoneView z, DParams P, const DMech *__restrict__ mech) {
+  const MechK m = mech_k(mech);
   const int X = z.mx + 2, Y = z.my + 2, Z = PLANE ? 1 : z.mz + 2;
   const int64_t t = (int64_t)blockIdx.x * kTB + threadIdx.x;
   if (t >= (int64_t)X * Y * Z) return;
@@ -693,7 +699,7 @@ __global__ void __launch_bounds__(kTB) k_properties(ZoneView z, DParams P, const
 #pragma unroll
     for (int l = 0; l < NS; ++l) {
       Yk[l] = z.sv[(int64_t)l * z.sz + p];
-      mwi += Yk[l] / m->mw[l];
+      mwi += Yk[l] * m->mw_inv[l];
       cpt += Yk[l] * cp[l];
       cvt += Yk[l] * (cp[l] - m->r_mw[l]);
     }
@@ -821,10 +827,11 @@ __global__ void k_copy1(const double *src, double *dst) { *dst = *src; }
 constexpr int kChemTB = 128;
 
 template <int NS>
-__global__ void __launch_bounds__(kChemTB) k_chem_batch(const DMech *__restrict__ m, int64_t n, int64_t count,
+__global__ void __launch_bounds__(kChemTB) k_chem_batch(const DMech *__restrict__ mech, int64_t n, int64_t count,
                                                         const int *__restrict__ idx, const double *__restrict__ rho_a,
                                                         const double *__restrict__ T_a, const double *__restrict__ Y_a,
                                                         double dt, double *__restrict__ dY, double *__restrict__ dT) {
+  const MechK m = mech_k(mech);
   extern __shared__ double sq_park[];
   const int64_t t = (int64_t)blockIdx.x * kChemTB + threadIdx.x;
   if (t >= count) return;
@@ -835,7 +842,7 @@ __global__ void __launch_bounds__(kChemTB) k_chem_batch(const DMech *__restrict_
   for (int l = 0; l < NS; ++l) Y[l] = Y_a[(int64_t)l * n + c];
   double mwi = 0;
 #pragma unroll
-  for (int l = 0; l < NS; ++l) mwi += Y[l] / m->mw[l];
+  for (int l = 0; l < NS; ++l) mwi += Y[l] * m->mw_inv[l];
   const double mw = 1 / mwi;
   const double p_old = rho * T * (kRuD / mw);
   d_enthalpy<NS>(T, m, h);
@@ -863,10 +870,11 @@ __global__ void __launch_bounds__(kChemTB) k_chem_batch(const DMech *__restrict_
 // state), by one-sided Jacobi rotations of its columns in FP64: the
 // conditioning of the point-implicit step, used as a training target.
 template <int NS>
-__global__ void __launch_bounds__(128) k_epi_sigma(const DMech *__restrict__ m, int64_t n,
+__global__ void __launch_bounds__(128) k_epi_sigma(const DMech *__restrict__ mech, int64_t n,
                                                    const double *__restrict__ rho_a, const double *__restrict__ T_a,
                                                    const double *__restrict__ Y_a, double dt,
                                                    double *__restrict__ sig) {
+  const MechK m = mech_k(mech);
   const int64_t c = (int64_t)blockIdx.x * 128 + threadIdx.x;
   if (c >= n) return;
   double Y[NS], om[NS], A[NS * NS];
@@ -938,8 +946,9 @@ __global__ void __launch_bounds__(kTB) k_chem_gather(ZoneView z, double *__restr
 }
 
 template <int NS>
-__global__ void __launch_bounds__(kTB) k_chem_scatter(ZoneView z, const DMech *__restrict__ m,
+__global__ void __launch_bounds__(kTB) k_chem_scatter(ZoneView z, const DMech *__restrict__ mech,
                                                       const double *__restrict__ dY, const double *__restrict__ dT) {
+  const MechK m = mech_k(mech);
   const int64_t t = (int64_t)blockIdx.x * kTB + threadIdx.x;
   const int64_t n = (int64_t)z.mx * z.my * z.mz;
   if (t >= n) return;
@@ -953,7 +962,7 @@ __global__ void __launch_bounds__(kTB) k_chem_scatter(ZoneView z, const DMech *_
     const double y = z.sv[(int64_t)l * z.sz + p] + dY[(int64_t)l * n + t];
     z.sv[(int64_t)l * z.sz + p] = y;
     z.cv[(int64_t)(5 + l) * z.sz + p] = rho * y;
-    mwi += y / m->mw[l];
+    mwi += y * m->mw_inv[l];
   }
   const double T = z.bv[5 * z.sz + p] + dT[t];
   z.bv[5 * z.sz + p] = T;
