@@ -434,8 +434,8 @@ int upload_mech(ostc_solver *s) {
       h.cp_ext[i] = c[0] + c[1] * t + c[2] * t2 + c[3] * t3 + c[4] * t4;
       h.h_ext[i] = c[0] * t + 0.5 * c[1] * t2 + c[2] * t3 / 3 + 0.25 * c[3] * t4 + 0.2 * c[4] * t5 + c[5] -
                    h.cp_ext[i] * t;
-      h.log_t_low[i] = std::log(t);
-      h.t_low_inv[i] = 1 / t;
+      h.g_ext[i] = c[0] * (1.0 - std::log(t)) - 0.5 * c[1] * t - c[2] * t2 / 6.0 - c[3] * t3 / 12.0 -
+                   c[4] * t4 * 0.05 + c[5] / t - c[6];
     }
     h.LJ_potent_inv[i] = m.LJ_potent_inv[i];
     h.log_LJ_potent_inv[i] = m.LJ_potent_inv[i] > 0 ? std::log(m.LJ_potent_inv[i]) : 0.0;
@@ -450,23 +450,48 @@ int upload_mech(ostc_solver *s) {
     h.log_kb_over_eps_jk[i] = m.kb_over_eps_jk[i] > 0 ? std::log(m.kb_over_eps_jk[i]) : 0.0;
   }
   for (int r = 0; r < nr; ++r) {
-    h.label[r] = m.label[r];
-    h.order[r] = m.order[r];
-    h.A[r] = m.A[r];
-    h.b[r] = m.b[r];
-    h.Ea[r] = m.Ea[r];
-    h.A2[r] = m.A2[r];
-    h.b2[r] = m.b2[r];
-    h.Ea2[r] = m.Ea2[r];
-    h.troe_alpha[r] = m.troe_alpha[r];
-    h.troe_t3[r] = m.troe_t3[r];
-    h.troe_t1[r] = m.troe_t1[r];
-    h.troe_t2[r] = m.troe_t2[r];
-  }
-  for (int i = 0; i < nr * ns; ++i) {
-    h.stoi_f[i] = m.stoi_f[i];
-    h.stoi_b[i] = m.stoi_b[i];
-    h.third_body_coeff[i] = m.third_body_coeff[i];
+    DMech::Reac &q = h.reac[r];
+    q.A = m.A[r];
+    q.b = m.b[r];
+    q.Ea = m.Ea[r];
+    q.A2 = m.A2[r];
+    q.b2 = m.b2[r];
+    q.Ea2 = m.Ea2[r];
+    q.alpha = m.troe_alpha[r];
+    q.t3_inv = 1 / m.troe_t3[r];
+    q.t1_inv = 1 / m.troe_t1[r];
+    q.t2 = m.troe_t2[r];
+    q.type = m.label[r];
+    q.order = m.order[r];
+    std::vector<int> side[2];
+    int ng = 0;
+    for (int &g : q.g) g = ns;
+    for (int l = 0; l < ns; ++l) {
+      const int i = r * ns + l, nf = m.stoi_f[i], nb = m.stoi_b[i];
+      h.stoi_f[i] = nf;
+      h.stoi_b[i] = nb;
+      h.nu_f[i] = nf;
+      h.nu_b[i] = nb;
+      h.nu[i] = nb - nf;
+      h.third_body_coeff[i] = m.third_body_coeff[i];
+      if (nf < 0 || nb < 0 || (nf != 0 && nb != 0)) q.more = 1;
+      if (nf != nb) {
+        if (ng == 4) {
+          q.more = 1;
+        } else {
+          q.g[ng] = l;
+          q.gc[ng++] = nb - nf;
+        }
+      }
+      for (int c = 0; c < nf && c < 3; ++c) side[0].push_back(l);
+      for (int c = 0; c < nb && c < 3; ++c) side[1].push_back(l);
+    }
+    if (side[0].size() > 2 || side[1].size() > 2) q.more = 1;
+    for (auto &v : side) v.resize(2, ns);
+    q.f0 = side[0][0];
+    q.f1 = side[0][1];
+    q.b0 = side[1][0];
+    q.b1 = side[1][1];
   }
   std::set<double> brk(m.t_low.begin(), m.t_low.begin() + ns);
   brk.insert(m.t_mid.begin(), m.t_mid.begin() + ns);
@@ -812,6 +837,7 @@ int ostc_init(const char *case_dir, int device, ostc_solver **out) {
   P.reaction = reaction;
   P.chemSrcMethod = p.get_int("chemSrcMethod", 0);
   P.nr = s->mech.n_reac;
+  P.last_inert = s->mech.last_inert() ? 1 : 0;
   P.inviscid_scheme = p.get_int("inviscid_scheme", 3);
   P.reconstruction = p.get_int("reconstruction", 2);
   P.limiter = p.get_int("limiter", 0);

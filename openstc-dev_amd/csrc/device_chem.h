@@ -38,9 +38,10 @@ __device__ inline double d_ipow(double x, int n) {
 template <int NS>
 __device__ inline void d_rate(MechK m, int r, double t, double lt, double it, const double *c,
                               const double *g, double temp_t, double &kf, double &kb) {
-  const int type = m->label[r];
-  double k = d_arrhenius(lt, it, m->A[r], m->b[r], m->Ea[r]);
-  if (type == 3) k += d_arrhenius(lt, it, m->A2[r], m->b2[r], m->Ea2[r]);
+  const auto &R = m->reac[r];
+  const int type = R.type;
+  double k = d_arrhenius(lt, it, R.A, R.b, R.Ea);
+  if (type == 3) k += d_arrhenius(lt, it, R.A2, R.b2, R.Ea2);
   if (type > 3) {
     double cc = 0;
 #pragma unroll
@@ -48,13 +49,13 @@ __device__ inline void d_rate(MechK m, int r, double t, double lt, double it, co
     if (type == 4) {
       k *= cc;
     } else {
-      const double klow = d_arrhenius(lt, it, m->A2[r], m->b2[r], m->Ea2[r]);
+      const double klow = d_arrhenius(lt, it, R.A2, R.b2, R.Ea2);
       const double khigh = k;
       const double pr = klow * cc / khigh;
       double F = 1.0;
       if (type > 5) {
-        double fc = (1 - m->troe_alpha[r]) * exp(-t / m->troe_t3[r]) + m->troe_alpha[r] * exp(-t / m->troe_t1[r]);
-        if (type == 7) fc += exp(-m->troe_t2[r] / t);
+        double fc = (1 - R.alpha) * exp(-t * R.t3_inv) + R.alpha * exp(-t * R.t1_inv);
+        if (type == 7) fc += exp(-R.t2 / t);
         const double lfc = log10(fc);
         const double c2 = -0.4 - 0.67 * lfc;
         const double nn = 0.75 - 1.27 * lfc;
@@ -70,98 +71,36 @@ __device__ inline void d_rate(MechK m, int r, double t, double lt, double it, co
   if (type == 0) {
     kb = 0;
   } else if (type == 2) {
-    kb = d_arrhenius(lt, it, m->A2[r], m->b2[r], m->Ea2[r]);
+    kb = d_arrhenius(lt, it, R.A2, R.b2, R.Ea2);
   } else {
     double dg = 0;
 #pragma unroll
     for (int l = 0; l < NS; ++l) dg += g[l] * (m->stoi_b[r * NS + l] - m->stoi_f[r * NS + l]);
-    const double kc = d_ipow(temp_t, m->order[r]) * exp(-dg);
+    const double kc = d_ipow(temp_t, R.order) * exp(-dg);
     kb = k / kc;
   }
 }
 
-// FiniteRateChem.cu:7-63 + 151-217: omega [kg/m3/s] and, when jac != null,
-// the exact-point-implicit Jacobian d omega_m / d(rho Y_n).  Rates, progress
-// and source are fused per reaction so no per-reaction array is kept.
-// omega_d (may be null): the destruction rates [kg/m3/s] of chemical_source.
-template <int NS>
-__device__ inline void d_chem_source(MechK m, double rho, double t, const double *Y, double *omega,
-                                     double *jac, double *omega_d = nullptr) {
-  double c[NS], g[NS];
-#pragma unroll
-  for (int l = 0; l < NS; ++l) c[l] = d_div(rho * Y[l], m->mw[l], m->mw_inv[l]) * 1e-3;
-  d_gibbs_rt<NS>(t, m, g);
-  const double temp_t = (kPatmD() / kRuD * 1e-3) / t;
-  const double lt = log(t), it = 1.0 / t;
-  const int nr = m->n_reac;
-  double creation[NS], destr[NS];
-#pragma unroll
-  for (int l = 0; l < NS; ++l) {
-    creation[l] = 0;
-    destr[l] = 0;
-  }
-  if (jac) {
-#pragma unroll
-    for (int a = 0; a < NS * NS; ++a) jac[a] = 0;
-  }
-  for (int r = 0; r < nr; ++r) {
-    double kf, kb;
-    d_rate<NS>(m, r, t, lt, it, c, g, temp_t, kf, kb);
-    double q1 = 1.0, q2 = 1.0;
-#pragma unroll
-    for (int l = 0; l < NS; ++l) {
-      q1 *= d_ipow(c[l], m->stoi_f[r * NS + l]);
-      q2 *= d_ipow(c[l], m->stoi_b[r * NS + l]);
-    }
-    q1 *= kf;
-    q2 = m->label[r] != 0 ? q2 * kb : 0.0;
-#pragma unroll
-    for (int l = 0; l < NS; ++l) {
-      const int nf = m->stoi_f[r * NS + l], nb = m->stoi_b[r * NS + l];
-      creation[l] += q2 * nf + q1 * nb;
-      destr[l] += q1 * nf + q2 * nb;
-    }
-    if (jac) {
-#pragma unroll
-      for (int n = 0; n < NS; ++n) {
-        const double dn = m->stoi_f[r * NS + n] * q1 - m->stoi_b[r * NS + n] * q2;
-#pragma unroll
-        for (int a = 0; a < NS; ++a) jac[a * NS + n] += (m->stoi_b[r * NS + a] - m->stoi_f[r * NS + a]) * dn;
-      }
-    }
-  }
-#pragma unroll
-  for (int l = 0; l < NS; ++l) omega[l] = creation[l] * (m->mw[l] * 1e+3) - destr[l] * (m->mw[l] * 1e+3);
-  if (omega_d)
-#pragma unroll
-    for (int l = 0; l < NS; ++l) omega_d[l] = destr[l] * (m->mw[l] * 1e+3);
-  if (jac) {
-#pragma unroll
-    for (int n = 0; n < NS; ++n) {
-      const bool on = Y[n] > 1e-25;
-#pragma unroll
-      for (int a = 0; a < NS; ++a) jac[a * NS + n] = on ? m->mw[a] * (jac[a * NS + n] / (rho * Y[n])) * 1e+3 : 0.0;
-    }
-  }
-}
-
-// The same source and Jacobian in two passes over the reactions, for kernels
-// that solve with I - dt J: the first computes omega and parks the rates of
+// Source and Jacobian of the chemistry batch in two passes over the
+// reactions: the first computes omega and parks the rates of
 // progress q1, q2 of reaction r at q[2r * stride], q[(2r + 1) * stride]
 // (LDS, one column per thread), the second accumulates the Jacobian from
 // them.  Keeping the 81 Jacobian sums out of the first pass (where the
 // concentrations, free energies and creation / destruction sums are live)
-// keeps the kernel in registers.  Sums run over r in the same order as in
-// d_chem_source, so the results are the same.
+// keeps the kernel in registers.
 template <int NS>
 __device__ inline void d_chem_rates(MechK m, double rho, double t, const double *Y, double *omega,
                                     double *q, int stride) {
   double c[NS], g[NS];
 #pragma unroll
   for (int l = 0; l < NS; ++l) c[l] = d_div(rho * Y[l], m->mw[l], m->mw_inv[l]) * 1e-3;
-  d_gibbs_rt<NS>(t, m, g);
   const double temp_t = (kPatmD() / kRuD * 1e-3) / t;
   const double lt = log(t), it = 1.0 / t;
+#pragma unroll
+  for (int l = 0; l < NS; ++l) {
+    if (l % 3 == 0) m = fresh(m);
+    g[l] = d_species_gibbs(m, l, t, lt, it);
+  }
   const int nr = m->n_reac;
   double creation[NS], destr[NS];
 #pragma unroll
@@ -179,7 +118,7 @@ __device__ inline void d_chem_rates(MechK m, double rho, double t, const double 
       q2 *= d_ipow(c[l], m->stoi_b[r * NS + l]);
     }
     q1 *= kf;
-    q2 = m->label[r] != 0 ? q2 * kb : 0.0;
+    q2 = m->reac[r].type != 0 ? q2 * kb : 0.0;
     q[2 * r * stride] = q1;
     q[(2 * r + 1) * stride] = q2;
 #pragma unroll
@@ -217,6 +156,225 @@ __device__ inline void d_epi_matrix(MechK m, double rho, const double *Y, double
       const double J = on ? m->mw[a] * (A[a * NS + n] / (rho * Y[n])) * 1e+3 : 0.0;
       A[a * NS + n] = EPI ? (a == n ? 1.0 : 0.0) - dt * J : J;
     }
+  }
+}
+
+// FiniteRateChem.cu:7-149 (+ 151-217 and 219-232): one pass over the
+// reactions giving omega [kg/m3/s] and, per WANT, nothing else (kOmega), the
+// sums S_an = sum_r (nu_b - nu_f)_a (nu_f q1 - nu_b q2)_n of the
+// exact-point-implicit Jacobian (kJacobian, row-major NA x NA, see
+// d_jacobian_entry), or the destruction rates (kDestruction).  q1, q2 are the
+// rates of progress: kf (Arrhenius + duplicate, third body, Lindemann, Troe)
+// and kb = kf / Kc (or the REV set, 0 if irreversible) times the
+// concentrations.
+//
+// NA: leading species that take part in reactions (NS, or NS - 1 when the
+// last one is inert: its row and column of the Jacobian are zero).
+// col: this thread's column (stride ld) of kinetics_slots(NS, WANT) pairs of
+// shared memory: concentration and g / RT of every species, (1, 0) for a
+// missing molecule, and with kJacobian and kDestruction the creation and
+// destruction sums.  A reaction addresses its species there by wave-uniform
+// index; only its owner reads a column, so there is no barrier.
+//
+// What bounds it: one wavefront is a long serial chain (about 40 exponentials),
+// so the time goes with its instructions and with how many wavefronts share a
+// SIMD.  Multiplying all NS powers of every reaction through scalar switches,
+// with integer coefficients converted in the loop, took 13,100 vector and
+// 6,200 scalar instructions per wavefront (9 species, 19 reactions, with the
+// solve) at one wavefront per SIMD and 40 % of the cycles in waits.  Indexed
+// species, coefficients read as double scalar operands and sums kept out of
+// registers leave 2 wavefronts per SIMD with the Jacobian, 4 without.
+enum Kinetics { kOmega, kJacobian, kDestruction };
+
+__host__ __device__ constexpr int kinetics_slots(int ns, int want) { return want == kOmega ? ns + 1 : 2 * ns + 2; }
+
+template <int NS, int NA, int WANT>
+__device__ inline void d_kinetics(MechK m, double rho, double t, const double *Y, double2 *col, int ld, double *omega,
+                                  double *out) {
+  const double lt = log(t), it = 1.0 / t;
+  double2 *sum = col + (NS + 1) * ld;  // (creation, destruction) of every species, one unused
+#pragma unroll
+  for (int l = 0; l < NS; ++l) {
+    m = fresh(m);
+    const double c = d_div(rho * Y[l], m->mw[l], m->mw_inv[l]) * 1e-3;
+    col[l * ld] = double2{c, d_species_gibbs(m, l, t, lt, it)};
+    if constexpr (WANT != kOmega) sum[l * ld] = double2{0.0, 0.0};
+  }
+  col[NS * ld] = double2{1.0, 0.0};
+  const double p0 = (kPatmD() / kRuD * 1e-3) / t;  // concentration at p_atm and T
+  if constexpr (WANT == kOmega) {
+#pragma unroll
+    for (int a = 0; a < NA; ++a) omega[a] = 0;
+  }
+  if constexpr (WANT == kJacobian) {
+#pragma unroll
+    for (int a = 0; a < NA * NA; ++a) out[a] = 0;
+  }
+  const int nr = m->n_reac;
+  for (int r = 0; r < nr; ++r) {
+    const auto &R = m->reac[r];
+    double q1 = col[R.f0 * ld].x * col[R.f1 * ld].x, q2 = col[R.b0 * ld].x * col[R.b1 * ld].x;
+    double dg = col[R.g[0] * ld].y * R.gc[0];
+#pragma unroll
+    for (int i = 1; i < 4; ++i) dg = fma(col[R.g[i] * ld].y, R.gc[i], dg);
+    const bool more = R.more != 0;
+    if (more) {
+      q1 = q2 = 1.0;
+      dg = 0;
+#pragma unroll 1
+      for (int l = 0; l < NS; ++l) {
+        const int nf = m->stoi_f[r * NS + l], nb = m->stoi_b[r * NS + l];
+        const double2 x = col[l * ld];
+        q1 *= d_ipow(x.x, nf);
+        q2 *= d_ipow(x.x, nb);
+        dg += x.y * (nb - nf);
+      }
+    }
+    const int type = R.type;
+    double k = d_arrhenius(lt, it, R.A, R.b, R.Ea);
+    if (type == 3) k += d_arrhenius(lt, it, R.A2, R.b2, R.Ea2);
+    if (type > 3) {
+      double cc = 0;
+#pragma unroll
+      for (int l = 0; l < NS; ++l) cc = fma(col[l * ld].x, m->third_body_coeff[r * NS + l], cc);
+      if (type == 4) {
+        k *= cc;
+      } else {
+        const double pr = d_arrhenius(lt, it, R.A2, R.b2, R.Ea2) * cc / k;
+        double F = 1.0;
+        if (type > 5) {
+          double fc = (1 - R.alpha) * exp(-t * R.t3_inv) + R.alpha * exp(-t * R.t1_inv);
+          if (type == 7) fc += exp(-R.t2 * it);
+          const double lfc = log10(fc);
+          const double lpr = log10(pr) + (-0.4 - 0.67 * lfc);
+          const double tempo = lpr / ((0.75 - 1.27 * lfc) - 0.14 * lpr);
+          F = exp(2.302585092994046 * (lfc / (1.0 + tempo * tempo)));
+        }
+        k = k * pr / (1.0 + pr) * F;
+      }
+    }
+    q1 *= k;
+    if (type == 0) {
+      q2 = 0;
+    } else if (type == 2) {
+      q2 *= d_arrhenius(lt, it, R.A2, R.b2, R.Ea2);
+    } else {
+      const int order = R.order;
+      double kc = exp(-dg);
+      if (order == 1)
+        kc *= p0;
+      else if (order != 0)
+        kc *= d_ipow(p0, order);
+      q2 *= k / kc;
+    }
+    if constexpr (WANT == kOmega) {
+      const double net = q1 - q2;
+#pragma unroll
+      for (int a = 0; a < NA; ++a) omega[a] = fma((double)m->nu[r * NS + a], net, omega[a]);
+    } else if (more) {
+#pragma unroll 1
+      for (int l = 0; l < NS; ++l) {
+        const double nf = m->nu_f[r * NS + l], nb = m->nu_b[r * NS + l];
+        double2 s = sum[l * ld];
+        s.x += q2 * nf + q1 * nb;
+        s.y += q1 * nf + q2 * nb;
+        sum[l * ld] = s;
+      }
+    } else {
+      // a species of the net list stands on one side: forward (gc < 0) or backward
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        double2 *s = sum + R.g[i] * ld;
+        const double c = R.gc[i], qc = c < 0 ? q2 : q1, qd = c < 0 ? q1 : q2;
+        double2 v = *s;
+        v.x = fma(fabs(c), qc, v.x);
+        v.y = fma(fabs(c), qd, v.y);
+        *s = v;
+      }
+    }
+    if constexpr (WANT == kJacobian) {
+      MechK mn = m;
+#pragma unroll
+      for (int n = 0; n < NA; ++n) {
+        if (n % 4 == 0) mn = fresh(mn);
+        const double dn = mn->nu_f[r * NS + n] * q1 - mn->nu_b[r * NS + n] * q2;
+#pragma unroll
+        for (int a = 0; a < NA; ++a) out[a * NA + n] = fma((double)m->nu[r * NS + a], dn, out[a * NA + n]);
+      }
+    }
+  }
+#pragma unroll
+  for (int a = 0; a < NA; ++a) {
+    if constexpr (WANT == kOmega) {
+      omega[a] *= m->mw[a] * 1e+3;
+    } else {
+      const double2 s = sum[a * ld];
+      omega[a] = (s.x - s.y) * (m->mw[a] * 1e+3);
+      if constexpr (WANT == kDestruction) out[a] = s.y * (m->mw[a] * 1e+3);
+    }
+  }
+}
+
+// d omega_a / d(rho Y_n) from the sum S_an: W_a 1e3 S_an / (rho Y_n), 0 where
+// species n is absent.  ry, iry: rho Y_n and its reciprocal.
+__device__ inline double d_jacobian_entry(double s, bool on, double ry, double iry, double mw) {
+  return on ? mw * d_div(s, ry, iry) * 1e+3 : 0.0;
+}
+
+__device__ inline void swap_double(double &a, double &b) {
+  uint2 x = __builtin_bit_cast(uint2, a), y = __builtin_bit_cast(uint2, b);
+  asm volatile("v_swap_b32 %0, %1" : "+v"(x.x), "+v"(y.x));
+  asm volatile("v_swap_b32 %0, %1" : "+v"(x.y), "+v"(y.y));
+  a = __builtin_bit_cast(double, x);
+  b = __builtin_bit_cast(double, y);
+}
+
+// x of A x = b for an N x N system held in registers, b overwritten:
+// elimination with row pivoting, the first largest entry of a column taken
+// (FiniteRateChem.cu:364-418 picks the same rows).  Only what later steps
+// read is swapped; a swap is a branch that a wavefront skips when none of its
+// cells takes that row, and the quotients of a column share the reciprocal of
+// its pivot (d_div rounds them like divisions).
+template <int N>
+__device__ inline void d_gauss_solve(double *A, double *b) {
+  double ip[N];
+#pragma unroll
+  for (int n = 0; n < N; ++n) {
+    int ik = n;
+    double best = fabs(A[n * N + n]);
+#pragma unroll
+    for (int r = n + 1; r < N; ++r) {
+      const double v = fabs(A[r * N + n]);
+      if (v > best) {
+        best = v;
+        ik = r;
+      }
+    }
+    // a register, not the N - n comparisons it came from
+    asm volatile("" : "+v"(ik));
+#pragma unroll
+    for (int r = n + 1; r < N; ++r) {
+      if (r == ik) {
+#pragma unroll
+        for (int c = n; c < N; ++c) swap_double(A[r * N + c], A[n * N + c]);
+        swap_double(b[r], b[n]);
+      }
+    }
+    const double piv = A[n * N + n];
+    ip[n] = 1.0 / piv;
+#pragma unroll
+    for (int r = n + 1; r < N; ++r) {
+      const double f = d_div(A[r * N + n], piv, ip[n]);
+#pragma unroll
+      for (int c = n + 1; c < N; ++c) A[r * N + c] = fma(-f, A[n * N + c], A[r * N + c]);
+      b[r] = fma(-f, b[n], b[r]);
+    }
+  }
+#pragma unroll
+  for (int r = N - 1; r >= 0; --r) {
+#pragma unroll
+    for (int c = r + 1; c < N; ++c) b[r] = fma(-A[r * N + c], b[c], b[r]);
+    b[r] = d_div(b[r], A[r * N + r], ip[r]);
   }
 }
 

@@ -16,11 +16,21 @@ constexpr int kMR = 50;   // reaction capacity of the device tables
 // live n_spec / n_reac.  Lives in device memory; kernels read it with
 // wave-uniform addresses.
 struct DMech {
+  // One reaction as the kinetics loop reads it: rate constants (1 / T3 and
+  // 1 / T1 of Troe's form), the species of the first two molecules of each
+  // side (n_spec: no such molecule), and the net coefficients nu_b - nu_f of
+  // the species that have one, ascending (g[i] with coefficient gc[i]).
+  // more: a side has further molecules or a species stands on both sides;
+  // stoi_f and stoi_b are walked instead.
+  struct Reac {
+    double A, b, Ea, A2, b2, Ea2, alpha, t3_inv, t1_inv, t2, gc[4];
+    int type, order, more, f0, f1, b0, b1, g[4], pad;
+  };
   int n_spec, n_reac;
   double mw[kMS], mw_inv[kMS], t_low[kMS], t_mid[kMS], hi[kMS * 7], lo[kMS * 7];
   // below t_low: cp / R stays cp(t_low) and h / R = h_ext + cp_ext T
   double cp_ext[kMS], h_ext[kMS];
-  double log_t_low[kMS], t_low_inv[kMS];
+  double g_ext[kMS];  // g / RT there, its value at t_low
   // the different t_low and t_mid of all species, ascending: between two of
   // them every species keeps its branch
   int n_brk;
@@ -28,10 +38,11 @@ struct DMech {
   double LJ_potent_inv[kMS], vis_coeff[kMS];
   double WjDivWi_to_One4th[kMS * kMS], sqrt_WiDivWjPl1Mul8[kMS * kMS];
   double binary_diffusivity_coeff[kMS * kMS], kb_over_eps_jk[kMS * kMS];
-  int label[kMR], stoi_f[kMR * kMS], stoi_b[kMR * kMS], order[kMR];
-  double A[kMR], b[kMR], Ea[kMR], A2[kMR], b2[kMR], Ea2[kMR];
-  double third_body_coeff[kMR * kMS];
-  double troe_alpha[kMR], troe_t3[kMR], troe_t1[kMR], troe_t2[kMR];
+  Reac reac[kMR];
+  int stoi_f[kMR * kMS], stoi_b[kMR * kMS];
+  // per reaction (rows of n_spec): forward and backward coefficients,
+  // nu_b - nu_f, third-body efficiencies
+  double nu_f[kMR * kMS], nu_b[kMR * kMS], nu[kMR * kMS], third_body_coeff[kMR * kMS];
   // logarithms of LJ_potent_inv and kb_over_eps_jk: the collision-integral
   // powers T*^-0.145 become exp(-0.145 (log T + log k))
   double log_LJ_potent_inv[kMS], log_kb_over_eps_jk[kMS * kMS];
@@ -50,6 +61,7 @@ struct DParams {
   double efix;  // Roe entropy-fix factor
   int turb_implicit, compress;  // SST: implicit source diagonal; compressibility correction 0-3
   int nr;                       // reactions of the mechanism (0 without chemistry)
+  int last_inert;               // the last species takes part in no reaction
   int jface;                    // HLLC / LF face vector (J0 m0 + J1 m1) / 2 (conservative metrics)
 };
 
@@ -130,6 +142,14 @@ __device__ inline double d_div(double a, double b, double rb) {
   return fma(fma(-b, q, a), rb, q);
 }
 
+// c ? a : b with both sides evaluated: left to itself the compiler turns a
+// choice between two polynomials into divergent branches that load their
+// coefficients inside, one scalar-load latency each
+__device__ inline double d_select(bool c, double a, double b) {
+  asm("" : "+v"(a), "+v"(b));
+  return c ? a : b;
+}
+
 // T and the weights of a0 .. a4 in h / R = a0 T + a1 T^2 / 2 + .. + a4 T^5 / 5 + a5
 struct TPow {
   double t, t2, t3, t4, p2, p3, p4, p5;
@@ -196,26 +216,18 @@ __device__ inline void d_cp(double t, MechK m, double *cp) {
   }
 }
 
-template <int NS>
-__device__ inline void d_gibbs_rt(double t, MechK m, double *g) {
-  const double log_t = log(t), t_inv = 1 / t;
-#pragma unroll
-  for (int i = 0; i < NS; ++i) {
-    if (i % 3 == 0) m = fresh(m);
-    // frozen at t_low below it
-    const bool cold = t < m->t_low[i];
-    const double x = cold ? (double)m->t_low[i] : t, x2 = x * x, x3 = x2 * x, x4 = x3 * x;
-    const double lx = cold ? (double)m->log_t_low[i] : log_t, xi = cold ? (double)m->t_low_inv[i] : t_inv;
-    auto poly = [&](double c0, double c1, double c2, double c3, double c4, double c5, double c6) {
-      return c0 * (1.0 - lx) - 0.5 * c1 * x - d_div(c2 * x2, 6.0, 1 / 6.0) - d_div(c3 * x3, 12.0, 1 / 12.0) -
-             c4 * x4 * 0.05 + c5 * xi - c6;
-    };
-    const auto *a = &m->lo[i * 7];
-    const auto *b = &m->hi[i * 7];
-    const double gl = poly(a[0], a[1], a[2], a[3], a[4], a[5], a[6]);
-    const double gh = poly(b[0], b[1], b[2], b[3], b[4], b[5], b[6]);
-    g[i] = cold || x < m->t_mid[i] ? gl : gh;
-  }
+// g_l / RT of species l at T (lt = ln T, it = 1 / T), frozen at t_low below it
+__device__ inline double d_species_gibbs(MechK m, int l, double t, double lt, double it) {
+  const double t2 = t * t, t3 = t2 * t, t4 = t3 * t;
+  auto poly = [&](double c0, double c1, double c2, double c3, double c4, double c5, double c6) {
+    return c0 * (1.0 - lt) - 0.5 * c1 * t - d_div(c2 * t2, 6.0, 1 / 6.0) - d_div(c3 * t3, 12.0, 1 / 12.0) -
+           c4 * t4 * 0.05 + c5 * it - c6;
+  };
+  const auto *a = &m->lo[l * 7];
+  const auto *b = &m->hi[l * 7];
+  const double gl = poly(a[0], a[1], a[2], a[3], a[4], a[5], a[6]);
+  const double gh = poly(b[0], b[1], b[2], b[3], b[4], b[5], b[6]);
+  return d_select(t < m->t_low[l], m->g_ext[l], d_select(t < m->t_mid[l], gl, gh));
 }
 
 // sum_l w_l h_l(T) and sum_l w_l cp_l(T) as one polynomial in T, its

@@ -32,6 +32,18 @@ hipError_t with_species(int ns, F &&f) {
   return with_mixture(ns, f);
 }
 
+// with_mixture plus the number of leading species that react, a second
+// integral constant: all of them, or all but the last when that one takes
+// part in no reaction (the bath gas)
+template <typename F>
+hipError_t with_kinetics(int ns, bool last_inert, F &&f) {
+  return with_mixture(ns, [&](auto c) {
+    constexpr int NS = decltype(c)::value;
+    if (last_inert) return f(c, std::integral_constant<int, NS - 1>{});
+    return f(c, c);
+  });
+}
+
 struct BCDesc {
   int type, face, dir;
   int rs[3], re[3];

@@ -63,6 +63,16 @@ struct Mechanism {
   std::vector<int> label, stoi_f, stoi_b, order;
   std::vector<double> A, b, Ea, A2, b2, Ea2, third_body_coeff;
   std::vector<double> troe_alpha, troe_t3, troe_t1, troe_t2;
+
+  // the last species takes part in no reaction
+  bool last_inert() const {
+    if (n_reac == 0) return false;
+    for (int r = 0; r < n_reac; ++r) {
+      const size_t i = (size_t)r * n_spec + n_spec - 1;
+      if (stoi_f[i] != 0 || stoi_b[i] != 0) return false;
+    }
+    return true;
+  }
 };
 
 // Atomic weight of an element symbol (upper case), -1 if unknown.

@@ -33,20 +33,22 @@ __device__ inline double wave_sum(double v) {
 
 // ------------------------------------------------------------- source
 // SourceTerm.cuh:11-37 (finite-rate part): dq = 0 for the flow components,
-// dq(5+l) = J omega_l, and the chemistry Jacobian (EPI) or its diagonal (DA).
+// dq(5+l) = J omega_l, and the chemistry Jacobian (METHOD 1, EPI) or its
+// diagonal (METHOD 2, DA; FiniteRateChem.cu:219-232: -omega_d / (rho Y)).
 // With accumulate (the SST kernel already initialised dq) the species rows
-// are added to and the flow rows left alone.  The EPI Jacobian is built in a
-// second pass over the rates of progress parked in LDS (one column per
-// thread, no barrier).  The park is dynamic LDS of 2 n_reac rows of kSrcTB
-// doubles, launched only with the EPI Jacobian: its size sets how many
-// workgroups share a CU (4 of them for 19 reactions, 2 waves per SIMD).
+// are added to and the flow rows left alone.  One instantiation per method:
+// the Jacobian's registers would otherwise set the occupancy of the explicit
+// source too (1 wavefront per SIMD where it has 4).  131,072 cells of 9 species
+// and 19 reactions: 127 -> 41 us; 20,503 cells: 63 -> 33 us; with the Jacobian,
+// 1.18 M cells: 1.37 -> 0.55 ms (0.9 GB of it, the Jacobian's stores).
 constexpr int kSrcTB = 128;
-constexpr int kParkMaxReac = 24;  // reactions per cell the LDS park holds
+constexpr int kMaxEpiReac = 24;  // reactions the point-implicit kernels accept
 
-template <int NS>
-__global__ void __launch_bounds__(kSrcTB) k_source(ZoneView z, DParams P, const DMech *__restrict__ mech, int accumulate) {
+template <int NS, int NA, int METHOD>
+__global__ void __launch_bounds__(kSrcTB, METHOD == 1 ? 2 : 3) k_source(ZoneView z, const DMech *__restrict__ mech,
+                                                                       int accumulate) {
   const MechK m = mech_k(mech);
-  extern __shared__ double sq_park[];
+  __shared__ double2 cg[kinetics_slots(NS, METHOD)][kSrcTB];
   const int64_t t = (int64_t)blockIdx.x * kSrcTB + threadIdx.x;
   const int64_t n = (int64_t)z.mx * z.my * z.mz;
   if (t >= n) return;
@@ -57,21 +59,28 @@ __global__ void __launch_bounds__(kSrcTB) k_source(ZoneView z, DParams P, const 
 #pragma unroll
   for (int l = 0; l < NS; ++l) Y[l] = z.sv[(int64_t)l * z.sz + p];
   const double rho = z.bv[p], T = z.bv[5 * z.sz + p], J = z.jac[p];
-  if (P.chemSrcMethod == 1) {
-    double jac[NS * NS];
-    d_chem_rates<NS>(m, rho, T, Y, om, sq_park + threadIdx.x, kSrcTB);
-    d_epi_matrix<NS, false>(m, rho, Y, 0.0, sq_park + threadIdx.x, kSrcTB, jac);
+  double2 *col = &cg[0][threadIdx.x];
+  if constexpr (METHOD == 1) {
+    double jac[NA * NA];
+    d_kinetics<NS, NA, kJacobian>(m, rho, T, Y, col, kSrcTB, om, jac);
 #pragma unroll
-    for (int c = 0; c < NS * NS; ++c) z.chem_jac[(int64_t)c * z.sz0 + q] = jac[c];
-  } else if (P.chemSrcMethod == 2) {
-    // FiniteRateChem.cu:219-232 diagonal approximation: -omega_d / (rho Y)
-    double od[NS];
-    d_chem_source<NS>(m, rho, T, Y, om, nullptr, od);
+    for (int c = 0; c < NS; ++c) {
+      const double ry = rho * Y[c], iry = 1.0 / ry;
 #pragma unroll
-    for (int l = 0; l < NS; ++l) z.chem_jac[(int64_t)l * z.sz0 + q] = Y[l] > 1e-25 ? -od[l] / (Y[l] * rho) : 0.0;
+      for (int a = 0; a < NS; ++a)
+        z.chem_jac[(int64_t)(a * NS + c) * z.sz0 + q] =
+            a < NA && c < NA ? d_jacobian_entry(jac[a * NA + c], Y[c] > 1e-25, ry, iry, m->mw[a]) : 0.0;
+    }
+  } else if constexpr (METHOD == 2) {
+    double od[NA];
+    d_kinetics<NS, NA, kDestruction>(m, rho, T, Y, col, kSrcTB, om, od);
+#pragma unroll
+    for (int l = 0; l < NS; ++l)
+      z.chem_jac[(int64_t)l * z.sz0 + q] = l < NA && Y[l] > 1e-25 ? -od[l] / (Y[l] * rho) : 0.0;
   } else {
-    d_chem_source<NS>(m, rho, T, Y, om, nullptr);
+    d_kinetics<NS, NA, kOmega>(m, rho, T, Y, col, kSrcTB, om, nullptr);
   }
+  for (int l = NA; l < NS; ++l) om[l] = 0;
   if (accumulate) {
 #pragma unroll
     for (int l = 0; l < NS; ++l) z.dq[(int64_t)(5 + l) * z.sz0 + q] += J * om[l];
@@ -837,32 +846,43 @@ __global__ void __launch_bounds__(kChemTB) k_chem_batch(const DMech *__restrict_
   if (t >= count) return;
   const int64_t c = idx ? (int64_t)idx[t] : t;
   const double rho = rho_a[c], T = T_a[c];
-  double Y[NS], om[NS], J[NS * NS], h[NS];
+  double Y[NS], om[NS], J[NS * NS];
 #pragma unroll
   for (int l = 0; l < NS; ++l) Y[l] = Y_a[(int64_t)l * n + c];
-  double mwi = 0;
-#pragma unroll
-  for (int l = 0; l < NS; ++l) mwi += Y[l] * m->mw_inv[l];
-  const double mw = 1 / mwi;
-  const double p_old = rho * T * (kRuD / mw);
-  d_enthalpy<NS>(T, m, h);
-  double rhoE = 0;
-#pragma unroll
-  for (int l = 0; l < NS; ++l) rhoE += h[l] * Y[l];
-  rhoE *= rho;
-  rhoE -= p_old;
   d_chem_rates<NS>(m, rho, T, Y, om, sq_park + threadIdx.x, kChemTB);
   d_epi_matrix<NS>(m, rho, Y, dt, sq_park + threadIdx.x, kChemTB, J);
   d_lu_solve<NS>(J, om);
   const double ri = 1.0 / rho;
-  double Yn[NS];
+  // sum Y_l h_l(T) of the old and the new composition, and the new one's cp:
+  // the first Newton step, which most cells need alone
+  double ho = 0, hn = 0, cp = 0, gas_o = 0, gas = 0;
+  const TPow tp(T);
+  MechK mk = m;
 #pragma unroll
-  for (int l = 0; l < NS; ++l) Yn[l] = ri * (rho * Y[l] + om[l] * dt);
-  double pn;
-  const double Tn = d_temperature<NS>(m, rho, rhoE, 0.0, 0.0, 0.0, Yn, T, pn);
-#pragma unroll
-  for (int l = 0; l < NS; ++l) dY[(int64_t)l * n + c] = Yn[l] - Y[l];
-  dT[c] = Tn - T;
+  for (int l = 0; l < NS; ++l) {
+    mk = fresh(mk);
+    const double h = d_species_h(mk, l, tp);
+    ho = fma(Y[l], h, ho);
+    gas_o = fma(Y[l], mk->r_mw[l], gas_o);
+    const double yn = ri * (rho * Y[l] + om[l] * dt);
+    dY[(int64_t)l * n + c] = yn - Y[l];
+    Y[l] = yn;
+    hn = fma(yn, h, hn);
+    cp = fma(yn, d_species_cp(mk, l, tp), cp);
+    gas = fma(yn, mk->r_mw[l], gas);
+  }
+  const double e = ho - gas_o * T;
+  double s = (hn - gas * T - e) / (cp - gas);
+  double tk = T - s, err = fabs(1 - tk / T);
+  MixPoly q;
+  q.ta = q.tb = 0;  // built in the loop
+  for (int iter = 1; err > 1e-3 && iter < 1000; ++iter) {
+    if (!q.holds(tk)) q.build<NS>(m, Y, tk);
+    s = (q.h(tk) - gas * tk - e) / (q.cp(tk) - gas);
+    err = fabs(1 - (tk - s) / tk);
+    tk -= s;
+  }
+  dT[c] = tk - T;
 }
 
 // Smallest singular value of the point-implicit matrix I - dt J of each cell
@@ -875,16 +895,20 @@ __global__ void __launch_bounds__(128) k_epi_sigma(const DMech *__restrict__ mec
                                                    const double *__restrict__ Y_a, double dt,
                                                    double *__restrict__ sig) {
   const MechK m = mech_k(mech);
+  __shared__ double2 cg[kinetics_slots(NS, kJacobian)][128];
   const int64_t c = (int64_t)blockIdx.x * 128 + threadIdx.x;
   if (c >= n) return;
   double Y[NS], om[NS], A[NS * NS];
 #pragma unroll
   for (int l = 0; l < NS; ++l) Y[l] = Y_a[(int64_t)l * n + c];
-  d_chem_source<NS>(m, rho_a[c], T_a[c], Y, om, A);
+  d_kinetics<NS, NS, kJacobian>(m, rho_a[c], T_a[c], Y, &cg[0][threadIdx.x], 128, om, A);
 #pragma unroll
-  for (int a = 0; a < NS; ++a)
+  for (int b = 0; b < NS; ++b) {
+    const double ry = rho_a[c] * Y[b], iry = 1.0 / ry;
 #pragma unroll
-    for (int b = 0; b < NS; ++b) A[a * NS + b] = (a == b ? 1.0 : 0.0) - dt * A[a * NS + b];
+    for (int a = 0; a < NS; ++a)
+      A[a * NS + b] = (a == b ? 1.0 : 0.0) - dt * d_jacobian_entry(A[a * NS + b], Y[b] > 1e-25, ry, iry, m->mw[a]);
+  }
   for (int sweep = 0; sweep < 12; ++sweep) {
     double off = 0;
 #pragma unroll
@@ -992,11 +1016,17 @@ hipError_t launch_chem_scatter(const ZoneView &z, const DParams &P, const DMech 
 
 hipError_t launch_source(const ZoneView &z, const DParams &P, const DMech *m, bool accumulate, hipStream_t s) {
   const int64_t n = (int64_t)z.mx * z.my * z.mz;
-  if (P.chemSrcMethod == 1 && (P.nr <= 0 || P.nr > kParkMaxReac)) return hipErrorInvalidValue;
-  const size_t park = P.chemSrcMethod == 1 ? (size_t)2 * P.nr * kSrcTB * sizeof(double) : 0;
-  return with_mixture(P.ns, [&](auto c) {
-    hipLaunchKernelGGL(k_source<decltype(c)::value>, dim3(nblk(n, kSrcTB)), dim3(kSrcTB), park, s, z, P, m,
-                       accumulate ? 1 : 0);
+  if (P.chemSrcMethod == 1 && (P.nr <= 0 || P.nr > kMaxEpiReac)) return hipErrorInvalidValue;
+  const dim3 g(nblk(n, kSrcTB)), b(kSrcTB);
+  return with_kinetics(P.ns, P.last_inert, [&](auto c, auto ca) {
+    constexpr int NS = decltype(c)::value, NA = decltype(ca)::value;
+    const int acc = accumulate ? 1 : 0;
+    if (P.chemSrcMethod == 1)
+      hipLaunchKernelGGL((k_source<NS, NA, 1>), g, b, 0, s, z, m, acc);
+    else if (P.chemSrcMethod == 2)
+      hipLaunchKernelGGL((k_source<NS, NA, 2>), g, b, 0, s, z, m, acc);
+    else
+      hipLaunchKernelGGL((k_source<NS, NA, 0>), g, b, 0, s, z, m, acc);
     return hipGetLastError();
   });
 }
@@ -1144,7 +1174,7 @@ hipError_t launch_copy_dt(const double *src, double *dst, hipStream_t s) {
 hipError_t launch_chem_batch(const DMech *m, int nr, int64_t n, const double *rho, const double *T, const double *Y,
                              double dt, double *dY, double *dT, hipStream_t s, int ns) {
   if (n <= 0) return hipSuccess;
-  if (nr <= 0 || nr > kParkMaxReac) return hipErrorInvalidValue;
+  if (nr <= 0 || nr > kMaxEpiReac) return hipErrorInvalidValue;
   const size_t park = (size_t)2 * nr * kChemTB * sizeof(double);
   return with_mixture(ns, [&](auto c) {
     hipLaunchKernelGGL(k_chem_batch<decltype(c)::value>, dim3(nblk(n, kChemTB)), dim3(kChemTB), park, s, m, n, n,
@@ -1164,7 +1194,7 @@ hipError_t launch_chem_batch_subset(const DMech *m, int nr, int64_t n, int64_t c
                                     const double *rho, const double *T, const double *Y, double dt, double *dY,
                                     double *dT, hipStream_t s) {
   if (count <= 0) return hipSuccess;
-  if (count > n || nr <= 0 || nr > kParkMaxReac) return hipErrorInvalidValue;
+  if (count > n || nr <= 0 || nr > kMaxEpiReac) return hipErrorInvalidValue;
   const size_t park = (size_t)2 * nr * kChemTB * sizeof(double);
   hipLaunchKernelGGL(k_chem_batch<9>, dim3(nblk(count, kChemTB)), dim3(kChemTB), park, s, m, n, count, idx, rho, T, Y,
                      dt, dY, dT);
