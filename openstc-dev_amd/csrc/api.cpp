@@ -64,6 +64,9 @@ struct Block {
   std::vector<InnerFace> inner;     // inner faces to other blocks, in file order
   std::vector<BoundaryFace> faces;
   std::vector<BCDesc> bcs;          // in application order
+  std::vector<BCGroup> bc_groups;   // the same as launches (group_bcs), descriptors in device memory
+  BCGroup wall_group;               // the wall ranges, for DPLUR
+  bool walls_inside = true;         // every wall range lies inside the block (DPLUR needs it)
   ZoneView z{};
   std::vector<void *> mem;
 };
@@ -707,7 +710,61 @@ int exchange_all(ostc_solver *s, bool with_cv) {
 
 int run_bcs(ostc_solver *s, Block &b, bool with_cv) {
   ostc_solver::Timer t(s, "boundary");
-  for (auto &bc : b.bcs) HIPCHK(launch_bc(b.z, s->P, s->d_mech, bc, with_cv, s->stream));
+  HIPCHK(launch_bcs(b.z, s->P, s->d_mech, b.bc_groups, with_cv, s->stream));
+  return 0;
+}
+
+// The boundary ranges of a block as launches: groups in order and the wall
+// ranges, their descriptors in one device array.
+int build_bc_groups(ostc_solver *s, Block &b) {
+  std::vector<BCDesc> live, walls;
+  for (const BCDesc &c : b.bcs) {
+    bool empty = false, inside = true;
+    const int m[3] = {b.mx, b.my, b.mz};
+    for (int x = 0; x < 3; ++x) {
+      empty = empty || c.re[x] < c.rs[x];
+      inside = inside && c.rs[x] >= 0 && c.re[x] < m[x];
+    }
+    if (empty) continue;
+    live.push_back(c);
+    if (c.type == BC_WALL) {
+      walls.push_back(c);
+      b.walls_inside = b.walls_inside && inside;
+    }
+  }
+  if (live.empty()) return 0;
+  std::vector<BCDesc> all;
+  // layers: threads per point of a range
+  auto add = [&](const std::vector<BCDesc> &d, int64_t layers, BCGroup &g) -> int {
+    int64_t wgs = 0;
+    for (const BCDesc &c : d) {
+      int64_t n = layers;
+      for (int x = 0; x < 3; ++x) n *= c.re[x] - c.rs[x] + 1;
+      if (n > ((int64_t)1 << 32) - kBcTB) return fail("boundary range has too many points");
+      all.push_back(c);
+      all.back().first = (unsigned)wgs;
+      wgs += (n + kBcTB - 1) / kBcTB;
+    }
+    if (wgs >= (int64_t)1 << 31) return fail("boundary ranges have too many points");
+    g.n = (int)d.size();
+    g.wgs = (unsigned)wgs;
+    return 0;
+  };
+  for (auto &d : group_bcs(live, b.z.g)) {
+    b.bc_groups.emplace_back();
+    if (add(d, b.z.g + 1, b.bc_groups.back())) return 1;
+  }
+  if (add(walls, 1, b.wall_group)) return 1;
+  void *p = nullptr;
+  HIPCHK(hipMalloc(&p, all.size() * sizeof(BCDesc)));
+  b.mem.push_back(p);
+  HIPCHK(hipMemcpy(p, all.data(), all.size() * sizeof(BCDesc), hipMemcpyHostToDevice));
+  const BCDesc *at = (const BCDesc *)p;
+  for (BCGroup &g : b.bc_groups) {
+    g.d = at;
+    at += g.n;
+  }
+  b.wall_group.d = at;
   return 0;
 }
 
@@ -1400,6 +1457,8 @@ int ostc_finalize(ostc_solver *s) {
       }
   }
   if (s->n_turb && compute_wall_distance(s)) return 1;
+  for (auto &b : s->blocks)
+    if (build_bc_groups(s, b)) return 1;
   // per-run scratch: partials, ticket counter, dt slot, residual scale
   s->w.max_blocks = (int)std::max<int64_t>((max_cells + 255) / 256 + 1, red_blocks);
   HIPCHK(hipMalloc(&s->w.partial, sizeof(double) * 4 * s->w.max_blocks));
@@ -1729,10 +1788,8 @@ static int implicit_block(ostc_solver *s, Block &b) {
   DParams P = s->P;
   if (s->chem_split) P.reaction = 0;
   if (method == 1) {
-    std::vector<BCDesc> walls;
-    for (auto &bc : b.bcs)
-      if (bc.type == BC_WALL) walls.push_back(bc);
-    HIPCHK(launch_dplur(b.z, P, s->d_mech, s->prm.get_int("DPLUR_inner_step", 3), walls, s->stream));
+    if (!b.walls_inside) return fail("DPLUR: a wall range reaches outside its block");
+    HIPCHK(launch_dplur(b.z, P, s->d_mech, s->prm.get_int("DPLUR_inner_step", 3), b.wall_group, s->stream));
   } else {
     HIPCHK(launch_chem_implicit(b.z, P, s->stream));
     if (s->n_turb && s->P.turb_implicit == 1) HIPCHK(launch_turb_implicit(b.z, s->P, s->stream));

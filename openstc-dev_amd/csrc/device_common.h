@@ -123,6 +123,12 @@ constexpr double kMwAirD = 28.9647;
 typedef const __attribute__((address_space(4))) DMech *MechK;
 __device__ inline MechK mech_k(const DMech *m) { return (MechK)m; }
 
+// Any table read at wave-uniform addresses that no kernel writes, the same way
+template <typename T>
+__device__ inline const __attribute__((address_space(4))) T *uniform_table(const T *p) {
+  return (const __attribute__((address_space(4))) T *)p;
+}
+
 // The mechanism pointer made opaque to the optimiser: a property evaluation
 // given fresh(m) loads its coefficients where it uses them (scalar-cache
 // hits) instead of sharing loads hoisted once and held in registers for the

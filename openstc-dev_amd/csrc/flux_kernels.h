@@ -54,7 +54,26 @@ struct BCDesc {
   double a_inf, gamma_inf, entropy, mw_inf;  // farfield state (rho..vel, sv above)
   double p_total, t_total, p_back;           // subsonic inflow (u, v, w: direction), back pressure
   double mut;                                // turbulent viscosity of the inflow / farfield state
+  unsigned first = 0;                        // first workgroup of this range in its launch
 };
+
+typedef const __attribute__((address_space(4))) BCDesc *BCDescK;
+
+// Boundary ranges in device memory that one launch handles: n descriptors
+// (n >= 1), wgs workgroups in all.
+struct BCGroup {
+  const BCDesc *d = nullptr;
+  int n = 0;
+  unsigned wgs = 0;
+};
+// Threads per workgroup of the kernels that walk a BCGroup
+constexpr int kBcTB = 256;
+// Ranges of one block, in application order, cut into groups that can run as
+// one launch each without changing the result: a range goes to the first
+// group after those of every earlier range that it meets, where two ranges
+// meet when one writes (the face layer and the g ghost layers) what the other
+// writes or reads (the face layer and g layers inwards).
+std::vector<std::vector<BCDesc>> group_bcs(const std::vector<BCDesc> &bcs, int g);
 
 // per-step scratch kept on the device so a run needs no host round trip
 struct StepScratch {
@@ -92,8 +111,9 @@ hipError_t launch_local_dt(const ZoneView &z, const DParams &P, const StepScratc
                            hipStream_t s);
 hipError_t launch_rk_update(const ZoneView &z, const DParams &P, const DMech *m, const double *dt, int rk,
                             hipStream_t s);
-hipError_t launch_bc(const ZoneView &z, const DParams &P, const DMech *m, const BCDesc &bc, bool with_cv,
-                     hipStream_t s);
+// the groups of one block in order; their descriptors lie in one array
+hipError_t launch_bcs(const ZoneView &z, const DParams &P, const DMech *m, const std::vector<BCGroup> &groups,
+                      bool with_cv, hipStream_t s);
 hipError_t launch_eliminate_k(const ZoneView &z, const DParams &P, bool with_cv, hipStream_t s);
 // k_planes_copied: a 2-D block whose k-ghost planes k_eliminate_k has just
 // made copies of k = 0 (then the k = 0 values are computed once)
@@ -131,9 +151,10 @@ hipError_t launch_chem_batch(const DMech *m, int nr, int64_t n, const double *rh
 // ---- steady path (implicit.hip)
 // point-implicit chemistry on dq with the local dt (EPI or DA per chemSrcMethod)
 hipError_t launch_chem_implicit(const ZoneView &z, const DParams &P, hipStream_t s);
-// DPLUR: dq0, inner sweeps (wall dq zeroed before each), dq back to dq/dt
-hipError_t launch_dplur(const ZoneView &z, const DParams &P, const DMech *m, int inner_steps,
-                        const std::vector<BCDesc> &walls, hipStream_t s);
+// DPLUR: dq0, inner sweeps (dq of the wall ranges zeroed before each; ranges
+// within the block), dq back to dq/dt
+hipError_t launch_dplur(const ZoneView &z, const DParams &P, const DMech *m, int inner_steps, const BCGroup &walls,
+                        hipStream_t s);
 // local-dt update of bv / sv from dq (cv untouched)
 hipError_t launch_update_bv(const ZoneView &z, const DParams &P, const DMech *m, hipStream_t s);
 // operator-split chemistry on a zone's interior: gather (rho, T, Y SoA with

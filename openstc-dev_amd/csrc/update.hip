@@ -309,11 +309,10 @@ __global__ void __launch_bounds__(kTB) k_inner_exchange(ZoneView z, ZoneView tz,
 // Lanes run along the face's fastest index: the layer for i-faces (ghosts
 // adjacent in memory), the point for j- and k-faces.
 template <int NS, bool WITH_CV>
-__global__ void __launch_bounds__(kTB) k_bc(ZoneView z, DParams P, const DMech *__restrict__ mech, BCDesc b) {
-  const MechK m = mech_k(mech);
+__device__ inline void bc_point(const ZoneView &z, const DParams &P, MechK m, BCDescK bp, uint32_t t) {
+  const auto &b = *bp;
   const int nx = b.re[0] - b.rs[0] + 1, ny = b.re[1] - b.rs[1] + 1, nz = b.re[2] - b.rs[2] + 1;
   const uint32_t npt = (uint32_t)nx * ny * nz, nl = z.g + 1;
-  const uint32_t t = blockIdx.x * kTB + threadIdx.x;
   if (t >= npt * nl) return;
   uint32_t pt, gl;
   if (b.face == 0) {
@@ -332,10 +331,7 @@ __global__ void __launch_bounds__(kTB) k_bc(ZoneView z, DParams P, const DMech *
   i += b.rs[0];
   j += b.rs[1];
   k += b.rs[2];
-  int d[3] = {0, 0, 0};
-  d[b.face] = b.dir;
-  const int64_t so[3] = {1, z.d2, z.d1};
-  const int64_t sd = d[0] * so[0] + d[1] * so[1] + d[2] * so[2];  // outward step
+  const int64_t sd = b.dir * (b.face == 0 ? 1 : b.face == 1 ? z.d2 : z.d1);  // outward step
   const int64_t p = z.at(i, j, k);
   double *bv = z.bv, *sv = z.sv;
   const int64_t S = z.sz;
@@ -649,6 +645,27 @@ __global__ void __launch_bounds__(kTB) k_bc(ZoneView z, DParams P, const DMech *
       if (WITH_CV) cv_point<NS>(z, m, pg, P.nt);
     }
   }
+}
+
+// the range that workgroup wg of a group belongs to
+__device__ inline BCDescK bc_of(BCDescK list, int n, unsigned wg) {
+  while (n > 1 && wg >= list[1].first) {
+    ++list;
+    --n;
+  }
+  return list;
+}
+
+// One launch takes every range of a group (group_bcs): a range alone has too
+// few points to fill the card, so its time is a launch and one chain of
+// dependent loads (4 to 5 us in air, 9 to 21 us with 9 species), whatever its
+// size.  Launches per application: mixing layer 5 -> 2, channel with its wall
+// partition 32 -> 3 (0.67 -> 0.10 ms).
+template <int NS, bool WITH_CV>
+__global__ void __launch_bounds__(kBcTB) k_bc(ZoneView z, DParams P, const DMech *__restrict__ mech,
+                                              const BCDesc *__restrict__ bcs, int n_bc) {
+  const BCDescK b = bc_of(uniform_table(bcs), n_bc, blockIdx.x);
+  bc_point<NS, WITH_CV>(z, P, mech_k(mech), b, (blockIdx.x - b->first) * kBcTB + threadIdx.x);
 }
 
 // FieldOperation.cuh:372-400 eliminate_k_gradient (2-D runs)
@@ -1052,18 +1069,51 @@ hipError_t launch_rk_update(const ZoneView &z, const DParams &P, const DMech *m,
   });
 }
 
-hipError_t launch_bc(const ZoneView &z, const DParams &P, const DMech *m, const BCDesc &bc, bool with_cv,
-                     hipStream_t s) {
-  const int64_t n = (int64_t)(bc.re[0] - bc.rs[0] + 1) * (bc.re[1] - bc.rs[1] + 1) * (bc.re[2] - bc.rs[2] + 1);
-  if (n <= 0) return hipSuccess;
-  if (n * (z.g + 1) > ((int64_t)1 << 32) - kTB) return hipErrorInvalidValue;  // 32-bit thread index
-  const dim3 g(nblk(n * (z.g + 1), kTB)), b(kTB);
+std::vector<std::vector<BCDesc>> group_bcs(const std::vector<BCDesc> &bcs, int g) {
+  struct Box {
+    int lo[3], hi[3];
+  };
+  auto box = [&](const BCDesc &b, int side) {  // the face layer and g layers outwards (side 1) or inwards (-1)
+    Box r;
+    for (int x = 0; x < 3; ++x) {
+      r.lo[x] = b.rs[x];
+      r.hi[x] = b.re[x];
+    }
+    if (side * b.dir > 0)
+      r.hi[b.face] += g;
+    else
+      r.lo[b.face] -= g;
+    return r;
+  };
+  auto meet = [](const Box &p, const Box &q) {
+    for (int x = 0; x < 3; ++x)
+      if (p.lo[x] > q.hi[x] || q.lo[x] > p.hi[x]) return false;
+    return true;
+  };
+  std::vector<std::vector<BCDesc>> groups;
+  std::vector<size_t> level(bcs.size(), 0);
+  for (size_t i = 0; i < bcs.size(); ++i) {
+    const Box w = box(bcs[i], 1), r = box(bcs[i], -1);
+    for (size_t j = 0; j < i; ++j) {
+      const Box wj = box(bcs[j], 1), rj = box(bcs[j], -1);
+      if (meet(w, wj) || meet(w, rj) || meet(r, wj)) level[i] = std::max(level[i], level[j] + 1);
+    }
+    if (level[i] >= groups.size()) groups.resize(level[i] + 1);
+    groups[level[i]].push_back(bcs[i]);
+  }
+  return groups;
+}
+
+hipError_t launch_bcs(const ZoneView &z, const DParams &P, const DMech *m, const std::vector<BCGroup> &groups,
+                      bool with_cv, hipStream_t s) {
   return with_species(P.ns, [&](auto c) {
     constexpr int NS = decltype(c)::value;
-    if (with_cv)
-      hipLaunchKernelGGL((k_bc<NS, true>), g, b, 0, s, z, P, m, bc);
-    else
-      hipLaunchKernelGGL((k_bc<NS, false>), g, b, 0, s, z, P, m, bc);
+    for (const BCGroup &g : groups) {
+      if (with_cv)
+        hipLaunchKernelGGL((k_bc<NS, true>), dim3(g.wgs), dim3(kBcTB), 0, s, z, P, m, g.d, g.n);
+      else
+        hipLaunchKernelGGL((k_bc<NS, false>), dim3(g.wgs), dim3(kBcTB), 0, s, z, P, m, g.d, g.n);
+    }
     return hipGetLastError();
   });
 }
