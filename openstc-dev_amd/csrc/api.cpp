@@ -65,6 +65,7 @@ struct Block {
   std::vector<BoundaryFace> faces;
   std::vector<BCDesc> bcs;          // in application order
   std::vector<BCGroup> bc_groups;   // the same as launches (group_bcs), descriptors in device memory
+  std::vector<BCGroup> bc_plane;    // 2-D: their k = 0 points only
   BCGroup wall_group;               // the wall ranges, for DPLUR
   bool walls_inside = true;         // every wall range lies inside the block (DPLUR needs it)
   ZoneView z{};
@@ -126,6 +127,7 @@ struct ostc_solver {
     (void)hipFree(w.res_scale);
     (void)hipFree(w.res_one);
     (void)hipFree(w.blk_dt);
+    (void)hipFree(w.dt_partial);
     for (auto &p : pending) {
       (void)hipEventDestroy(p.a);
       (void)hipEventDestroy(p.b);
@@ -708,9 +710,10 @@ int exchange_all(ostc_solver *s, bool with_cv) {
   return 0;
 }
 
-int run_bcs(ostc_solver *s, Block &b, bool with_cv) {
+// plane: the k = 0 points of a 2-D block alone
+int run_bcs(ostc_solver *s, Block &b, bool with_cv, bool plane = false) {
   ostc_solver::Timer t(s, "boundary");
-  HIPCHK(launch_bcs(b.z, s->P, s->d_mech, b.bc_groups, with_cv, s->stream));
+  HIPCHK(launch_bcs(b.z, s->P, s->d_mech, plane ? b.bc_plane : b.bc_groups, with_cv, s->stream));
   return 0;
 }
 
@@ -754,16 +757,29 @@ int build_bc_groups(ostc_solver *s, Block &b) {
     b.bc_groups.emplace_back();
     if (add(d, b.z.g + 1, b.bc_groups.back())) return 1;
   }
+  if (s->P.dim == 2) {
+    std::vector<BCDesc> plane;
+    for (BCDesc c : live) {
+      if (c.face == 2 || c.rs[2] > 0 || c.re[2] < 0) continue;
+      c.rs[2] = c.re[2] = 0;
+      plane.push_back(c);
+    }
+    for (auto &d : group_bcs(plane, b.z.g)) {
+      b.bc_plane.emplace_back();
+      if (add(d, b.z.g + 1, b.bc_plane.back())) return 1;
+    }
+  }
   if (add(walls, 1, b.wall_group)) return 1;
   void *p = nullptr;
   HIPCHK(hipMalloc(&p, all.size() * sizeof(BCDesc)));
   b.mem.push_back(p);
   HIPCHK(hipMemcpy(p, all.data(), all.size() * sizeof(BCDesc), hipMemcpyHostToDevice));
   const BCDesc *at = (const BCDesc *)p;
-  for (BCGroup &g : b.bc_groups) {
-    g.d = at;
-    at += g.n;
-  }
+  for (auto *list : {&b.bc_groups, &b.bc_plane})
+    for (BCGroup &g : *list) {
+      g.d = at;
+      at += g.n;
+    }
   b.wall_group.d = at;
   return 0;
 }
@@ -792,11 +808,12 @@ int rhs_block(ostc_solver *s, Block &b, bool *dt_done = nullptr) {
   return 0;
 }
 
-// k_planes_copied: in 2-D, k_eliminate_k ran right before (the k-ghost
-// planes hold copies of k = 0)
-int properties_block(ostc_solver *s, Block &b, bool k_planes_copied) {
+// k_planes_copied: in 2-D, the k-ghost planes hold (or will hold) copies of
+// k = 0; the others as launch_properties takes them
+int properties_block(ostc_solver *s, Block &b, bool k_planes_copied, bool ghosts = true, double *dt_partial = nullptr,
+                     bool store_dt = false) {
   ostc_solver::Timer t(s, "properties");
-  HIPCHK(launch_properties(b.z, s->P, s->d_mech, k_planes_copied, s->stream));
+  HIPCHK(launch_properties(b.z, s->P, s->d_mech, k_planes_copied, s->stream, ghosts, dt_partial, store_dt));
   return 0;
 }
 
@@ -806,8 +823,9 @@ int global_dt_device(ostc_solver *s) {
   ostc_solver::Timer t(s, "local_dt");
   const int nb = (int)s->blocks.size();
   for (int bi = 0; bi < nb; ++bi)
-    HIPCHK(launch_local_dt(s->blocks[bi].z, s->P, s->w, nb == 1 ? s->w.dt : s->w.blk_dt + bi, s->stream));
-  if (nb > 1) HIPCHK(launch_min_of(s->w.blk_dt, nb, s->w.dt, s->stream));
+    HIPCHK(launch_local_dt(s->blocks[bi].z, s->P, s->w, nb == 1 ? s->w.dt : s->w.blk_dt + bi, s->stream,
+                           nb == 1 ? s->w.dt_copy : nullptr));
+  if (nb > 1) HIPCHK(launch_min_of(s->w.blk_dt, nb, s->w.dt, s->stream, s->w.dt_copy));
   return 0;
 }
 
@@ -1463,6 +1481,7 @@ int ostc_finalize(ostc_solver *s) {
   s->w.max_blocks = (int)std::max<int64_t>((max_cells + 255) / 256 + 1, red_blocks);
   HIPCHK(hipMalloc(&s->w.partial, sizeof(double) * 4 * s->w.max_blocks));
   HIPCHK(hipMalloc(&s->w.blk_dt, sizeof(double) * s->blocks.size()));
+  HIPCHK(hipMalloc(&s->w.dt_partial, sizeof(double) * kMaxDtPartials));
   HIPCHK(hipMalloc(&s->w.counter, sizeof(unsigned)));
   HIPCHK(hipMemsetAsync(s->w.counter, 0, sizeof(unsigned), s->stream));
   HIPCHK(hipMalloc(&s->w.dt, sizeof(double)));
@@ -1711,6 +1730,15 @@ int ostc_step_rk3(ostc_solver *s, int nsteps, double *dt_hist, double *res_hist)
   const double fixed_dt = s->prm.get_real("dt", 1e-5);
   const int os = std::max(1, s->prm.get_int("output_screen", 1));
   int rc = 0;
+  // A lone 2-D block: only the k = 0 plane is computed on, its k-ghost planes
+  // are copies that nothing reads before the call ends, so they are written by
+  // the last stage alone.  Its properties pass also gives the next stage's
+  // time step (not with SST, whose mu_t of that stage enters it), when the
+  // update's workgroups can each reduce the partial minima (kMaxDtPartials).
+  const bool plane = s->P.dim == 2 && s->blocks.size() == 1 && s->blocks[0].mz == 1 && s->blocks[0].inner.empty();
+  const bool plane_dt = plane && !fixed && s->n_turb == 0 &&
+                        properties_dt_blocks(s->blocks[0].z) <= kMaxDtPartials;
+  bool dt_ready = false;  // dt_partial holds the coming stage's time steps
   auto body = [&]() -> int {
     if (fixed) HIPCHK(hipMemcpyAsync(s->w.dt, &fixed_dt, sizeof(double), hipMemcpyHostToDevice, s->stream));
     for (int it = 0; it < nsteps; ++it) {
@@ -1720,25 +1748,33 @@ int ostc_step_rk3(ostc_solver *s, int nsteps, double *dt_hist, double *res_hist)
         // qn: stage 0 of k_rk_update stores the step's initial state
       }
       for (int rk = 0; rk < 3; ++rk) {
+        const int to_go = 3 * (nsteps - it) - rk - 1;  // stages after this one
+        s->w.dt_copy = d_dt + it * 3 + rk;
         // one block: the k-sweep computes the CFL dt where it can
         bool dt_done = false;
-        const bool fold_dt = !fixed && s->blocks.size() == 1;
+        const bool fold_dt = !fixed && s->blocks.size() == 1 && !dt_ready;
         for (auto &b : s->blocks)
           if (rhs_block(s, b, fold_dt ? &dt_done : nullptr)) return 1;
-        if (!fixed && !dt_done && global_dt_device(s)) return 1;
-        HIPCHK(launch_copy_dt(s->w.dt, d_dt + it * 3 + rk, s->stream));
+        if (fixed)
+          HIPCHK(launch_copy_dt(s->w.dt, s->w.dt_copy, s->stream));
+        else if (!dt_ready && !dt_done && global_dt_device(s))
+          return 1;
+        const bool ghosts = !plane || to_go == 0;  // the k-ghost planes are brought up to date
         for (auto &b : s->blocks) {
           {
             ostc_solver::Timer t(s, "rk_update");
-            HIPCHK(launch_rk_update(b.z, s->P, s->d_mech, s->w.dt, rk, s->stream));
+            HIPCHK(launch_rk_update(b.z, s->P, s->d_mech, s->w.dt, rk, s->stream, dt_ready ? s->w.dt_partial : nullptr,
+                                    properties_dt_blocks(b.z), s->w.dt_copy));
           }
-          if (run_bcs(s, b, true)) return 1;
+          if (run_bcs(s, b, true, !ghosts)) return 1;
         }
         if (exchange_all(s, true)) return 1;
-        if (s->P.dim == 2)
-          for (auto &b : s->blocks) HIPCHK(launch_eliminate_k(b.z, s->P, true, s->stream));
+        // the last stage's boundary ranges read the planes that the stage before left
+        if (s->P.dim == 2 && (ghosts || to_go == 1))
+          for (auto &b : s->blocks) HIPCHK(launch_eliminate_k(b.z, s->P, true, s->stream, !ghosts));
+        dt_ready = plane_dt && to_go > 0;
         for (auto &b : s->blocks)
-          if (properties_block(s, b, true)) return 1;
+          if (properties_block(s, b, true, ghosts, dt_ready ? s->w.dt_partial : nullptr, to_go == 1)) return 1;
       }
       if (step % os == 0 || step == 1) {
         ostc_solver::Timer t(s, "residual");

@@ -319,10 +319,11 @@ __device__ inline double d_temperature(MechK m, double rho, double rhoE, double 
 // TimeAdvanceFunc.cuh:50-100: the CFL time step of the cell at point p
 // (interior index q): the inviscid spectral radii of the three directions
 // plus the viscous radius.  The inviscid radii are kept per direction when
-// the zone stores them (z.inv_sr, for DPLUR).  One definition for the
-// stand-alone pass and for the sweep that computes it on the way.
-template <int MIX>
-__device__ inline double cell_dt(const ZoneView &z, const DParams &P, int64_t p, int64_t q) {
+// the zone stores them (z.inv_sr, for DPLUR).  a, gamma, mul: sound speed,
+// specific-heat ratio and viscosity of the point.  One definition for the
+// stand-alone pass and for the kernels that compute it on the way.
+__device__ inline double cell_dt(const ZoneView &z, const DParams &P, int64_t p, int64_t q, double a, double gamma,
+                                 double mul) {
   double mm[9];
 #pragma unroll
   for (int c = 0; c < 9; ++c) mm[c] = z.metric[c * z.sz + p];
@@ -333,7 +334,6 @@ __device__ inline double cell_dt(const ZoneView &z, const DParams &P, int64_t p,
   const double U = u * mm[0] + v * mm[1] + w * mm[2];
   const double V = u * mm[3] + v * mm[4] + w * mm[5];
   const double W = u * mm[6] + v * mm[7] + w * mm[8];
-  const double a = z.acoustic[p];
   const double r0 = fabs(U) + a * gxi, r1 = fabs(V) + a * geta;
   const double r2 = P.dim == 3 ? fabs(W) + a * gzeta : 0.0;
   const double sri = r0 + r1 + r2;
@@ -342,14 +342,19 @@ __device__ inline double cell_dt(const ZoneView &z, const DParams &P, int64_t p,
     z.inv_sr[z.sz0 + q] = r1;
     z.inv_sr[2 * z.sz0 + q] = r2;
   }
-  const double gamma = MIX ? z.gam[p] : kGam;
   const double c1 = fmax(gamma, 4.0 / 3.0) / z.bv[p];
-  double c2 = z.mul[p] / P.Pr;
+  double c2 = mul / P.Pr;
   if (z.mut) c2 += z.mut[p] / P.Prt;
   double srv = gxi * gxi + geta * geta;
   if (P.dim == 3) srv += gzeta * gzeta;
   srv *= c1 * c2;
   return P.cfl / (sri + srv);
+}
+
+// the same with the stored properties of the point
+template <int MIX>
+__device__ inline double cell_dt(const ZoneView &z, const DParams &P, int64_t p, int64_t q) {
+  return cell_dt(z, P, p, q, z.acoustic[p], MIX ? z.gam[p] : kGam, z.mul[p]);
 }
 
 }  // namespace ostc

@@ -1536,7 +1536,7 @@ static int sweep_segments(int per_cu, int cross, int n, int rows) {
 template <int NS, int NT, int SCHEME, typename R>
 static hipError_t launch_sweep_t(const ZoneView &z, const DParams &P, const DMech *m, int dir, bool init,
                                  hipStream_t s, double *dt_partial = nullptr, double *dt_out = nullptr,
-                                 int max_partials = 0, bool *dt_done = nullptr) {
+                                 int max_partials = 0, bool *dt_done = nullptr, double *dt_copy = nullptr) {
   if (dir == 0) {
     const int64_t waves = ((int64_t)z.my * (z.mx + 1) + 62) / 63;
     const int bpp = (int)((waves + 3) / 4);
@@ -1584,7 +1584,7 @@ static hipError_t launch_sweep_t(const ZoneView &z, const DParams &P, const DMec
                          dt_partial);
       hipError_t e = hipGetLastError();
       if (e != hipSuccess) return e;
-      e = launch_min_of(dt_partial, (int)gr.x, dt_out, s);
+      e = launch_min_of(dt_partial, (int)gr.x, dt_out, s, dt_copy);
       if (e == hipSuccess && dt_done) *dt_done = true;
       return e;
     } else {

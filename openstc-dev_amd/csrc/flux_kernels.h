@@ -75,6 +75,10 @@ constexpr int kBcTB = 256;
 // writes or reads (the face layer and g layers inwards).
 std::vector<std::vector<BCDesc>> group_bcs(const std::vector<BCDesc> &bcs, int g);
 
+// partial minima of the time step that every workgroup of the update reduces
+// for itself: 4 loads a thread
+constexpr int kMaxDtPartials = 1024;
+
 // per-step scratch kept on the device so a run needs no host round trip
 struct StepScratch {
   double *partial;         // per-block partials (>= 4 * max_blocks)
@@ -85,6 +89,8 @@ struct StepScratch {
   double *res_scale;       // 4
   double *res_one;         // 5: the residual of one ostc_residual call
   double *blk_dt;          // one CFL minimum per block (multi-block cases)
+  double *dt_partial;      // per-workgroup CFL minima that k_properties leaves for the next stage (kMaxDtPartials)
+  double *dt_copy;         // second place of the stage's CFL minimum (its history slot), may be null
   int max_blocks;
   int hist_cap;            // steps dt_hist / res_hist hold (grows, never shrinks)
 };
@@ -108,17 +114,22 @@ hipError_t launch_flux_sweep_sst(const ZoneView &z, const DParams &P, const DMec
 // finite-rate source; accumulate: add to dq (already initialised by launch_sst)
 hipError_t launch_source(const ZoneView &z, const DParams &P, const DMech *m, bool accumulate, hipStream_t s);
 hipError_t launch_local_dt(const ZoneView &z, const DParams &P, const StepScratch &w, double *dt_out,
-                           hipStream_t s);
-hipError_t launch_rk_update(const ZoneView &z, const DParams &P, const DMech *m, const double *dt, int rk,
-                            hipStream_t s);
+                           hipStream_t s, double *copy = nullptr);
+// partial (non-null): *dt = *copy = min(partial[0..nb)) first
+hipError_t launch_rk_update(const ZoneView &z, const DParams &P, const DMech *m, double *dt, int rk, hipStream_t s,
+                            const double *partial = nullptr, int nb = 0, double *copy = nullptr);
 // the groups of one block in order; their descriptors lie in one array
 hipError_t launch_bcs(const ZoneView &z, const DParams &P, const DMech *m, const std::vector<BCGroup> &groups,
                       bool with_cv, hipStream_t s);
-hipError_t launch_eliminate_k(const ZoneView &z, const DParams &P, bool with_cv, hipStream_t s);
-// k_planes_copied: a 2-D block whose k-ghost planes k_eliminate_k has just
-// made copies of k = 0 (then the k = 0 values are computed once)
+// rim: only the points that boundary ranges read (within g of the edges)
+hipError_t launch_eliminate_k(const ZoneView &z, const DParams &P, bool with_cv, hipStream_t s, bool rim = false);
+// k_planes_copied: a 2-D block whose k-ghost planes hold copies of k = 0 (then
+// the k = 0 values are computed once, and stored on the ghost planes k = -1, 1
+// with ghosts); dt_partial: also the smallest time step of each of the
+// properties_dt_blocks workgroups, the cells' own in dt_local with store_dt
 hipError_t launch_properties(const ZoneView &z, const DParams &P, const DMech *m, bool k_planes_copied,
-                             hipStream_t s);
+                             hipStream_t s, bool ghosts = true, double *dt_partial = nullptr, bool store_dt = false);
+int properties_dt_blocks(const ZoneView &z);
 hipError_t launch_velocity(const ZoneView &z, hipStream_t s);
 hipError_t launch_cv_from_bv(const ZoneView &z, const DParams &P, const DMech *m, hipStream_t s);
 hipError_t launch_store_last(const ZoneView &z, hipStream_t s);
@@ -131,7 +142,7 @@ hipError_t launch_residual_blocks(const std::vector<const ZoneView *> &zs, const
                                   hipStream_t s, double *out = nullptr);
 hipError_t launch_copy_dt(const double *src, double *dst, hipStream_t s);
 // *out = min(in[0..n)) (n >= 1)
-hipError_t launch_min_of(const double *in, int n, double *out, hipStream_t s);
+hipError_t launch_min_of(const double *in, int n, double *out, hipStream_t s, double *copy = nullptr);
 // inner-face exchange of block z with target tz (DataCommunication.cuh:58-110)
 hipError_t launch_inner_exchange(const ZoneView &z, const ZoneView &tz, const DParams &P, const DMech *m,
                                  const InnerFaceDesc &f, bool with_cv, hipStream_t s);

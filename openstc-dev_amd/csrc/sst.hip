@@ -49,7 +49,9 @@ __global__ void __launch_bounds__(kTB) k_wall_distance(ZoneView z, const double 
 
 // central point gradient 0.5 (xi_c dF/di + eta_c dF/dj + zeta_c dF/dk)
 __device__ inline void point_grad(const ZoneView &z, const double *f, int64_t p, const double *mm, double *g) {
-  const double di = f[p + 1] - f[p - 1], dj = f[p + z.d2] - f[p - z.d2], dk = f[p + z.d1] - f[p - z.d1];
+  // in 2-D the k-ghost planes are copies of k = 0, refreshed at the end of a run
+  const double di = f[p + 1] - f[p - 1], dj = f[p + z.d2] - f[p - z.d2];
+  const double dk = z.mz > 1 ? f[p + z.d1] - f[p - z.d1] : 0.0;
 #pragma unroll
   for (int c = 0; c < 3; ++c) g[c] = 0.5 * (mm[c] * di + mm[3 + c] * dj + mm[6 + c] * dk);
 }

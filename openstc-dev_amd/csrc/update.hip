@@ -123,27 +123,50 @@ __global__ void __launch_bounds__(kTB) k_local_dt(ZoneView z, DParams P, double 
   }
 }
 
-__global__ void __launch_bounds__(kTB) k_min_final(const double *partial, int nb, double *out) {
+// minimum of partial[0..nb) in every thread of a workgroup of kTB
+__device__ inline double block_min(const double *partial, int nb) {
   double r = 1e+6;
   for (int b = threadIdx.x; b < nb; b += kTB) r = fmin(r, partial[b]);
   __shared__ double sm[kTB / 64];
   r = wave_min(r);
   if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = r;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    double b = sm[0];
+  r = sm[0];
 #pragma unroll
-    for (int w = 1; w < kTB / 64; ++w) b = fmin(b, sm[w]);
-    *out = b;
+  for (int w = 1; w < kTB / 64; ++w) r = fmin(r, sm[w]);
+  return r;
+}
+
+// copy (may be null): a second place for the result
+__global__ void __launch_bounds__(kTB) k_min_final(const double *partial, int nb, double *out, double *copy) {
+  const double r = block_min(partial, nb);
+  if (threadIdx.x == 0) {
+    *out = r;
+    if (copy) *copy = r;
   }
 }
 
 // ------------------------------------------------------------- RK update
 // RK.cuh:10-14 (SSP-RK3 a, b, c) and RK.cuh:197-253 update_cv_and_bv_rk.
+// With partial, the stage's time step is the minimum of its nb values, which
+// every workgroup takes for itself (nb is small: k_properties of a 2-D block)
+// and the first one leaves in dt and copy: a launch less than a reduction
+// kernel, which takes 2 to 5 us whatever it reduces.
 template <int NS>
 __global__ void __launch_bounds__(kTB) k_rk_update(ZoneView z, DParams P, const DMech *__restrict__ mech,
-                                                    const double *__restrict__ dtp, int rk) {
+                                                    double *dtp, int rk, const double *__restrict__ partial, int nb,
+                                                    double *copy) {
   const MechK m = mech_k(mech);
+  double dt;
+  if (partial) {
+    dt = block_min(partial, nb);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      *dtp = dt;
+      *copy = dt;
+    }
+  } else {
+    dt = *dtp;
+  }
   const int64_t t = (int64_t)blockIdx.x * kTB + threadIdx.x;
   const int64_t n = (int64_t)z.mx * z.my * z.mz;
   if (t >= n) return;
@@ -153,7 +176,7 @@ __global__ void __launch_bounds__(kTB) k_rk_update(ZoneView z, DParams P, const 
   const double B = rk == 0 ? 0.0 : (rk == 1 ? 0.25 : 2.0 / 3.0);
   const double C = rk == 0 ? 1.0 : (rk == 1 ? 0.25 : 2.0 / 3.0);
   const int64_t p = z.at(i, j, k), q = z.at0(i, j, k);
-  const double dtj = *dtp / z.jac[p];
+  const double dtj = dt / z.jac[p];
   constexpr int NV = 5 + NS;
   double cv[NV];
   // stage 0 keeps the step's initial state in qn on the way (the stages
@@ -668,14 +691,16 @@ __global__ void __launch_bounds__(kBcTB) k_bc(ZoneView z, DParams P, const DMech
   bc_point<NS, WITH_CV>(z, P, mech_k(mech), b, (blockIdx.x - b->first) * kBcTB + threadIdx.x);
 }
 
-// FieldOperation.cuh:372-400 eliminate_k_gradient (2-D runs)
+// FieldOperation.cuh:372-400 eliminate_k_gradient (2-D runs).  rim: only the
+// points within g of the block's edges (ghosts included).
 template <bool WITH_CV>
-__global__ void __launch_bounds__(kTB) k_eliminate_k(ZoneView z, DParams P) {
+__global__ void __launch_bounds__(kTB) k_eliminate_k(ZoneView z, DParams P, int rim) {
   const int X = z.mx + 2 * z.g, Y = z.my + 2 * z.g;
   const int64_t t = (int64_t)blockIdx.x * kTB + threadIdx.x;
   if (t >= (int64_t)X * Y) return;
   const uint32_t jj = (uint32_t)t / (uint32_t)X;
   const int i = (int)((uint32_t)t - jj * (uint32_t)X) - z.g, j = (int)jj - z.g;
+  if (rim && i > z.g && i < z.mx - 1 - z.g && j > z.g && j < z.my - 1 - z.g) return;
   const int64_t p0 = z.at(i, j, 0);
   for (int k = 1; k <= z.g; ++k) {
     const int64_t pu = p0 + k * z.d1, pd = p0 - k * z.d1;
@@ -700,18 +725,22 @@ __global__ void __launch_bounds__(kTB) k_eliminate_k(ZoneView z, DParams P) {
 }
 
 // FieldOperation.cuh:112-146 update_physical_properties on [-1, m].  PLANE:
-// a 2-D block, whose k-ghost planes the preceding k_eliminate_k made copies
-// of k = 0 (bv and every scalar): the k = 0 values are computed once and
-// stored on k = -1, 0, 1 (bit-identical to computing each plane), the Mach
-// number from each plane's own |u|.
+// a 2-D block, whose k-ghost planes hold copies of k = 0 (bv and every
+// scalar): the k = 0 values are computed once and, with ghosts, stored on
+// k = -1, 0, 1 (bit-identical to computing each plane), the Mach number from
+// each plane's own |u|.  With dt_partial (PLANE), each workgroup also leaves
+// the smallest time step of its interior cells there (k_rk_update reduces
+// them), the cells' own in dt_local when store_dt is set.
 template <int NS, bool PLANE>
-__global__ void __launch_bounds__(kTB) k_properties(ZoneView z, DParams P, const DMech *__restrict__ mech) {
+__global__ void __launch_bounds__(kTB) k_properties(ZoneView z, DParams P, const DMech *__restrict__ mech, int ghosts,
+                                                    double *dt_partial, int store_dt) {
   const MechK m = mech_k(mech);
   const int X = z.mx + 2, Y = z.my + 2, Z = PLANE ? 1 : z.mz + 2;
   const int64_t t = (int64_t)blockIdx.x * kTB + threadIdx.x;
-  if (t >= (int64_t)X * Y * Z) return;
+  const bool live = t < (int64_t)X * Y * Z;
+  if (!PLANE && !live) return;
   int i, j, k;
-  unflatten3(t, X, Y, i, j, k);
+  unflatten3(live ? t : 0, X, Y, i, j, k);  // a thread past the end repeats the first point and stores nothing
   --i;
   --j;
   k = PLANE ? 0 : k - 1;
@@ -740,7 +769,8 @@ __global__ void __launch_bounds__(kTB) k_properties(ZoneView z, DParams P, const
     mu = d_sutherland(T);
     lam = mu * cp / P.Pr;
   }
-  for (int kk = PLANE ? -1 : 0; kk <= (PLANE ? 1 : 0); ++kk) {
+  const int planes = PLANE && ghosts ? 1 : 0;
+  for (int kk = live ? -planes : planes + 1; kk <= planes; ++kk) {
     const int64_t q = p + kk * z.d1;
     if constexpr (NS > 0) {
       z.cp[q] = cpt;
@@ -752,6 +782,24 @@ __global__ void __launch_bounds__(kTB) k_properties(ZoneView z, DParams P, const
     z.mul[q] = mu;
     z.cond[q] = lam;
     z.mach[q] = z.vel[q] / a;
+  }  if constexpr (PLANE) {
+    if (!dt_partial) return;
+    double best = 1e+6;
+    if (live && i >= 0 && i < z.mx && j >= 0 && j < z.my) {
+      const int64_t q = z.at0(i, j, 0);
+      const double dtl = cell_dt(z, P, p, q, a, NS > 0 ? gam : kGam, mu);
+      if (store_dt) z.dt_local[q] = dtl;
+      best = fmin(best, dtl);
+    }
+    __shared__ double sm[kTB / 64];
+    best = wave_min(best);
+    if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = best;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+#pragma unroll
+      for (int w = 1; w < kTB / 64; ++w) best = fmin(best, sm[w]);
+      dt_partial[blockIdx.x] = best;
+    }
   }
 }
 
@@ -1048,7 +1096,8 @@ hipError_t launch_source(const ZoneView &z, const DParams &P, const DMech *m, bo
   });
 }
 
-hipError_t launch_local_dt(const ZoneView &z, const DParams &P, const StepScratch &w, double *dt_out, hipStream_t s) {
+hipError_t launch_local_dt(const ZoneView &z, const DParams &P, const StepScratch &w, double *dt_out, hipStream_t s,
+                           double *copy) {
   const int64_t n = (int64_t)z.mx * z.my * z.mz;
   const int nb = (int)std::min<int64_t>(kRedBlocks, nblk(n, kTB));
   if (nb > w.max_blocks) return hipErrorInvalidValue;
@@ -1056,15 +1105,16 @@ hipError_t launch_local_dt(const ZoneView &z, const DParams &P, const StepScratc
     hipLaunchKernelGGL(k_local_dt<1>, dim3(nb), dim3(kTB), 0, s, z, P, w.partial);
   else
     hipLaunchKernelGGL(k_local_dt<0>, dim3(nb), dim3(kTB), 0, s, z, P, w.partial);
-  hipLaunchKernelGGL(k_min_final, dim3(1), dim3(kTB), 0, s, (const double *)w.partial, nb, dt_out);
+  hipLaunchKernelGGL(k_min_final, dim3(1), dim3(kTB), 0, s, (const double *)w.partial, nb, dt_out, copy);
   return hipGetLastError();
 }
 
-hipError_t launch_rk_update(const ZoneView &z, const DParams &P, const DMech *m, const double *dt, int rk,
-                            hipStream_t s) {
+hipError_t launch_rk_update(const ZoneView &z, const DParams &P, const DMech *m, double *dt, int rk, hipStream_t s,
+                            const double *partial, int nb, double *copy) {
   const int64_t n = (int64_t)z.mx * z.my * z.mz;
   return with_species(P.ns, [&](auto c) {
-    hipLaunchKernelGGL(k_rk_update<decltype(c)::value>, dim3(nblk(n, kTB)), dim3(kTB), 0, s, z, P, m, dt, rk);
+    hipLaunchKernelGGL(k_rk_update<decltype(c)::value>, dim3(nblk(n, kTB)), dim3(kTB), 0, s, z, P, m, dt, rk, partial,
+                       nb, copy);
     return hipGetLastError();
   });
 }
@@ -1118,29 +1168,31 @@ hipError_t launch_bcs(const ZoneView &z, const DParams &P, const DMech *m, const
   });
 }
 
-hipError_t launch_eliminate_k(const ZoneView &z, const DParams &P, bool with_cv, hipStream_t s) {
+hipError_t launch_eliminate_k(const ZoneView &z, const DParams &P, bool with_cv, hipStream_t s, bool rim) {
   const int64_t n = (int64_t)(z.mx + 2 * z.g) * (z.my + 2 * z.g);
   if (with_cv)
-    hipLaunchKernelGGL(k_eliminate_k<true>, dim3(nblk(n, kTB)), dim3(kTB), 0, s, z, P);
+    hipLaunchKernelGGL(k_eliminate_k<true>, dim3(nblk(n, kTB)), dim3(kTB), 0, s, z, P, rim ? 1 : 0);
   else
-    hipLaunchKernelGGL(k_eliminate_k<false>, dim3(nblk(n, kTB)), dim3(kTB), 0, s, z, P);
+    hipLaunchKernelGGL(k_eliminate_k<false>, dim3(nblk(n, kTB)), dim3(kTB), 0, s, z, P, rim ? 1 : 0);
   return hipGetLastError();
 }
 
 hipError_t launch_properties(const ZoneView &z, const DParams &P, const DMech *m, bool k_planes_copied,
-                             hipStream_t s) {
+                             hipStream_t s, bool ghosts, double *dt_partial, bool store_dt) {
   const bool plane = k_planes_copied && P.dim == 2 && z.mz == 1;
   const int64_t n = (int64_t)(z.mx + 2) * (z.my + 2) * (plane ? 1 : z.mz + 2);
   const dim3 g(nblk(n, kTB)), b(kTB);
   return with_species(P.ns, [&](auto c) {
     constexpr int NS = decltype(c)::value;
     if (plane)
-      hipLaunchKernelGGL((k_properties<NS, true>), g, b, 0, s, z, P, m);
+      hipLaunchKernelGGL((k_properties<NS, true>), g, b, 0, s, z, P, m, ghosts ? 1 : 0, dt_partial, store_dt ? 1 : 0);
     else
-      hipLaunchKernelGGL((k_properties<NS, false>), g, b, 0, s, z, P, m);
+      hipLaunchKernelGGL((k_properties<NS, false>), g, b, 0, s, z, P, m, 0, (double *)nullptr, 0);
     return hipGetLastError();
   });
 }
+
+int properties_dt_blocks(const ZoneView &z) { return (int)nblk((int64_t)(z.mx + 2) * (z.my + 2), kTB); }
 
 hipError_t launch_velocity(const ZoneView &z, hipStream_t s) {
   const int64_t n = (int64_t)(z.mx + 2 * z.g) * (z.my + 2 * z.g) * (z.mz + 2 * z.g);
@@ -1211,8 +1263,8 @@ hipError_t launch_inner_exchange(const ZoneView &z, const ZoneView &tz, const DP
   });
 }
 
-hipError_t launch_min_of(const double *in, int n, double *out, hipStream_t s) {
-  hipLaunchKernelGGL(k_min_final, dim3(1), dim3(kTB), 0, s, in, n, out);
+hipError_t launch_min_of(const double *in, int n, double *out, hipStream_t s, double *copy) {
+  hipLaunchKernelGGL(k_min_final, dim3(1), dim3(kTB), 0, s, in, n, out, copy);
   return hipGetLastError();
 }
 
