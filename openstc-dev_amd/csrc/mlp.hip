@@ -9,8 +9,15 @@
 // accumulation for split-K weight gradients).
 //
 // Tile: 64 x 64 outputs per workgroup of 4 wavefronts (each 32 x 32 = 2 x 2
-// MFMA tiles), K step 32.  LDS rows are padded to 40 BF16 (80 B) so the 16-B
-// fragment reads of a wavefront spread over the banks.
+// MFMA tiles), K step 64, the next step's operands loaded into registers
+// while the current one is multiplied.  The products of a mini-batch are
+// short (K = 24 to 264 forward, one 300-row share of the batch backward), so
+// a tile's time is a few global-load latencies: K steps of 32 that waited for
+// their own loads, with LDS moved in 2-byte pieces, took 13 / 17 / 20 us for
+// the forward, input-gradient and weight-gradient products of 8,192 rows;
+// this takes 10.5 / 15.5 / 14.0 us.
+// LDS rows are 68 BF16 long: the 8-byte reads of a fragment and the 4-byte
+// writes of a transposed operand (two K rows paired) spread over the banks.
 //
 // MFMA 16x16x32 BF16 operand layout (lane l of a wave64):
 //   A fragment: row l%16, k = 8*(l/16) + 0..7
@@ -18,6 +25,7 @@
 //   C/D f32x4 : col l%16, row = 4*(l/16) + 0..3
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 
 #include "mlp.h"
@@ -26,22 +34,87 @@ namespace ostc {
 
 namespace {
 
-constexpr int BM = 64, BN = 64, BK = 32, LDK = 40;
+constexpr int BM = 64, BN = 64, BK = 64, LDK = 68;
 
 __device__ inline __bf16 to_bf(float x) { return (__bf16)x; }
 __device__ inline float from_bf(__bf16 x) { return (float)x; }
 
+typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2;
+typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
 
+// eight consecutive values as one or two 16-byte loads (launch_gemm checks
+// the alignment)
 template <typename T>
-__device__ inline void load8(const T *p, float *v) {
+struct Oct;
+template <>
+struct Oct<float> {
+  f32x4 lo, hi;
+  __device__ void load(const float *p) {
+    lo = *(const f32x4 *)p;
+    hi = *(const f32x4 *)(p + 4);
+  }
+  __device__ void clear() { lo = hi = f32x4{0.f, 0.f, 0.f, 0.f}; }
+  __device__ __bf16 bf(int e) const { return to_bf(e < 4 ? lo[e & 3] : hi[e & 3]); }
+};
+template <>
+struct Oct<__bf16> {
+  bf16x8 v;
+  __device__ void load(const __bf16 *p) { v = *(const bf16x8 *)p; }
+  __device__ void clear() {
 #pragma unroll
-  for (int e = 0; e < 8; ++e) v[e] = (float)p[e];
-}
+    for (int e = 0; e < 8; ++e) v[e] = (__bf16)0.f;
+  }
+  __device__ __bf16 bf(int e) const { return v[e]; }
+};
+
+// One operand's 64 x 64 tile, 16 values a thread: rows of the tile are the
+// operand's M (or N) index, columns its K index.  KMAJOR: stored K x M, M
+// contiguous -- the thread holds 8 values of two adjacent K rows and writes
+// them in pairs; otherwise M x K, K contiguous.
+template <typename T>
+struct TileLoader {
+  Oct<T> a, b;
+
+  __device__ void load(bool kmajor, const T *p, int ld, int m0, int M, int k0, int k1, int tid) {
+    a.clear();
+    b.clear();
+    if (!kmajor) {
+      const int m = m0 + (tid >> 2), k = k0 + (tid & 3) * 16;
+      if (m < M) {
+        const T *q = p + (int64_t)m * ld + k;
+        if (k < k1) a.load(q);
+        if (k + 8 < k1) b.load(q + 8);
+      }
+    } else {
+      const int k = k0 + (tid >> 3) * 2, m = m0 + (tid & 7) * 8;
+      if (m < M) {
+        const T *q = p + (int64_t)k * ld + m;
+        if (k < k1) a.load(q);
+        if (k + 1 < k1) b.load(q + ld);
+      }
+    }
+  }
+
+  __device__ void store(bool kmajor, __bf16 (*t)[LDK], int tid) const {
+    if (!kmajor) {
+      __bf16 *q = &t[tid >> 2][(tid & 3) * 16];
+#pragma unroll
+      for (int e = 0; e < 8; e += 4) {
+        *(bf16x4 *)(q + e) = bf16x4{a.bf(e), a.bf(e + 1), a.bf(e + 2), a.bf(e + 3)};
+        *(bf16x4 *)(q + 8 + e) = bf16x4{b.bf(e), b.bf(e + 1), b.bf(e + 2), b.bf(e + 3)};
+      }
+    } else {
+      const int k = (tid >> 3) * 2, m = (tid & 7) * 8;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) *(bf16x2 *)&t[m + e][k] = bf16x2{a.bf(e), b.bf(e)};
+    }
+  }
+};
 
 template <typename TA, typename TB>
 __global__ void __launch_bounds__(256) k_gemm(GemmArgs g, const TA *__restrict__ A, const TB *__restrict__ B) {
-  __shared__ __bf16 As[BM][LDK];
-  __shared__ __bf16 Bs[BN][LDK];
+  __shared__ __attribute__((aligned(16))) __bf16 As[BM][LDK];
+  __shared__ __attribute__((aligned(16))) __bf16 Bs[BN][LDK];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
   const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
@@ -49,79 +122,44 @@ __global__ void __launch_bounds__(256) k_gemm(GemmArgs g, const TA *__restrict__
   // (chunks are whole K steps so every 8-element load stays 16-byte aligned)
   const int kchunk = (((g.K + (int)gridDim.z - 1) / (int)gridDim.z) + BK - 1) / BK * BK;
   const int kz0 = blockIdx.z * kchunk, kz1 = min(g.K, kz0 + kchunk);
+  const bool ka = g.transA != 0, kb = g.transB == 0;  // operand stored with K as its row
   f32x4 acc[2][2];
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
     for (int b = 0; b < 2; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-
+  TileLoader<TA> la;
+  TileLoader<TB> lb;
+  if (kz0 < kz1) {
+    la.load(ka, A, g.lda, m0, g.M, kz0, kz1, tid);
+    lb.load(kb, B, g.ldb, n0, g.N, kz0, kz1, tid);
+  }
   for (int k0 = kz0; k0 < kz1; k0 += BK) {
-    // ---- stage A tile (64 x 32) ----
-    {
-      float v[8];
-      if (!g.transA) {  // A stored M x K (lda), k contiguous
-        const int m = tid >> 2, kk = (tid & 3) * 8;
-        const int gm = m0 + m, gk = k0 + kk;
-        if (gm < g.M && gk < kz1)
-          load8(A + (int64_t)gm * g.lda + gk, v);
-        else
-#pragma unroll
-          for (int e = 0; e < 8; ++e) v[e] = 0.f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) As[m][kk + e] = (gk + e < kz1) ? to_bf(v[e]) : to_bf(0.f);
-      } else {  // A stored K x M (lda), m contiguous
-        const int k = tid >> 3, mm = (tid & 7) * 8;
-        const int gk = k0 + k, gm = m0 + mm;
-        if (gk < kz1 && gm < g.M)
-          load8(A + (int64_t)gk * g.lda + gm, v);
-        else
-#pragma unroll
-          for (int e = 0; e < 8; ++e) v[e] = 0.f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) As[mm + e][k] = (gm + e < g.M) ? to_bf(v[e]) : to_bf(0.f);
-      }
-    }
-    // ---- stage B tile (32 x 64), held as Bs[n][k] ----
-    {
-      float v[8];
-      if (!g.transB) {  // B stored K x N (ldb), n contiguous
-        const int k = tid >> 3, nn = (tid & 7) * 8;
-        const int gk = k0 + k, gn = n0 + nn;
-        if (gk < kz1 && gn < g.N)
-          load8(B + (int64_t)gk * g.ldb + gn, v);
-        else
-#pragma unroll
-          for (int e = 0; e < 8; ++e) v[e] = 0.f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) Bs[nn + e][k] = (gn + e < g.N) ? to_bf(v[e]) : to_bf(0.f);
-      } else {  // B stored N x K (ldb), k contiguous
-        const int n = tid >> 2, kk = (tid & 3) * 8;
-        const int gn = n0 + n, gk = k0 + kk;
-        if (gn < g.N && gk < kz1)
-          load8(B + (int64_t)gn * g.ldb + gk, v);
-        else
-#pragma unroll
-          for (int e = 0; e < 8; ++e) v[e] = 0.f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) Bs[n][kk + e] = (gk + e < kz1) ? to_bf(v[e]) : to_bf(0.f);
-      }
-    }
+    la.store(ka, As, tid);
+    lb.store(kb, Bs, tid);
     __syncthreads();
-    bf16x8 af[2], bfr[2];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int r = wm * 32 + t * 16 + (lane & 15);
-      const int c = wn * 32 + t * 16 + (lane & 15);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        af[t][e] = As[r][8 * (lane >> 4) + e];
-        bfr[t][e] = Bs[c][8 * (lane >> 4) + e];
-      }
+    if (k0 + BK < kz1) {
+      la.load(ka, A, g.lda, m0, g.M, k0 + BK, kz1, tid);
+      lb.load(kb, B, g.ldb, n0, g.N, k0 + BK, kz1, tid);
     }
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+    for (int ks = 0; ks < BK; ks += 32) {
+      bf16x8 af[2], bfr[2];
 #pragma unroll
-      for (int b = 0; b < 2; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[a], bfr[b], acc[a][b], 0, 0, 0);
+      for (int t = 0; t < 2; ++t) {
+        const __bf16 *ra = &As[wm * 32 + t * 16 + (lane & 15)][ks + 8 * (lane >> 4)];
+        const __bf16 *rb = &Bs[wn * 32 + t * 16 + (lane & 15)][ks + 8 * (lane >> 4)];
+        const bf16x4 a0 = *(const bf16x4 *)ra, a1 = *(const bf16x4 *)(ra + 4);
+        const bf16x4 b0 = *(const bf16x4 *)rb, b1 = *(const bf16x4 *)(rb + 4);
+        af[t] = __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
+        bfr[t] = __builtin_shufflevector(b0, b1, 0, 1, 2, 3, 4, 5, 6, 7);
+      }
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+          acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[a], bfr[b], acc[a][b], 0, 0, 0);
+    }
     __syncthreads();
   }
 
@@ -166,6 +204,7 @@ hipError_t launch_gemm(const GemmArgs &g, const void *A, bool a_bf16, const void
   if (g.ldc < g.N || (!g.Cf && !g.Cb)) return hipErrorInvalidValue;
   if (g.mode == EPI_ATOMIC && !g.Cf) return hipErrorInvalidValue;
   if (g.mode == EPI_GELU_GRAD && !g.Zin) return hipErrorInvalidValue;
+  if (((uintptr_t)A | (uintptr_t)B) % 16) return hipErrorInvalidValue;
   if (split_k < 1) split_k = 1;
   if (split_k > 1 && g.mode != EPI_ATOMIC) return hipErrorInvalidValue;
   const dim3 grid((g.N + BN - 1) / BN, (g.M + BM - 1) / BM, split_k), blk(256);
@@ -198,17 +237,19 @@ __global__ void k_fill_cols_bf16(__bf16 *__restrict__ dst, int64_t rows, int col
 }
 
 // MSE over the first nout of ld columns: loss = sum (y - t)^2 / (M nout),
-// G = d loss / d y (zero in the padding columns)
+// G = d loss / d y (zero in the padding columns).  At most kMseBlocks
+// workgroups, since each adds its share to one address and those additions
+// queue up (8,192 x 16: 512 workgroups 8.5 us, 64 6.4 us)
+constexpr int kMseBlocks = 64;
 __global__ void k_mse(const float *__restrict__ Y, const float *__restrict__ T, int M, int nout, int ld,
                       float *__restrict__ G, float *__restrict__ loss_acc) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   float l = 0.f;
-  if (i < (int64_t)M * ld) {
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < (int64_t)M * ld; i += (int64_t)gridDim.x * 256) {
     const int c = (int)(i % ld);
     float g = 0.f;
     if (c < nout) {
       const float d = Y[i] - T[i];
-      l = d * d;
+      l += d * d;
       g = 2.f * d / ((float)M * (float)nout);
     }
     G[i] = g;
@@ -264,7 +305,7 @@ hipError_t launch_fill_cols_bf16(__bf16 *dst, int64_t rows, int cols, int c0, co
 
 hipError_t launch_mse(const float *Y, const float *T, int M, int nout, int ld, float *G, float *loss_acc,
                       hipStream_t s) {
-  hipLaunchKernelGGL(k_mse, dim3(nb((int64_t)M * ld)), dim3(256), 0, s, Y, T, M, nout, ld, G, loss_acc);
+  hipLaunchKernelGGL(k_mse, dim3(std::min<unsigned>(kMseBlocks, nb((int64_t)M * ld))), dim3(256), 0, s, Y, T, M, nout, ld, G, loss_acc);
   return hipGetLastError();
 }
 

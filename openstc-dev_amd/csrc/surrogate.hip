@@ -163,6 +163,15 @@ __global__ void k_pack_x(int64_t B, const float *__restrict__ x, __bf16 *__restr
   write_x_row(X, r, xs);
 }
 
+// host-supplied targets [B x 8] -> rows of kYld, zero padded
+__global__ void k_pack_t(int64_t B, const float *__restrict__ t, float *__restrict__ T) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= B * kYld) return;
+  const int64_t r = i / kYld;
+  const int c = (int)(i - r * kYld);
+  T[i] = c < kSurOut ? t[r * kSurOut + c] : 0.f;
+}
+
 // standardised network inputs of cells c0 .. c0+count
 __global__ void k_sur_features(const DMech *__restrict__ mech, int64_t n, int64_t c0, int64_t count,
                                const double *__restrict__ rho, const double *__restrict__ T,
@@ -672,6 +681,7 @@ struct SurrogateState {
   // training workspace for batches up to tcap rows
   int64_t tcap = 0;
   __bf16 *tX = nullptr, *tH[3] = {};
+  float *tIn = nullptr;  // a host batch as it came: inputs, then targets
   float *tT = nullptr, *tZ[3] = {}, *tY = nullptr, *tG = nullptr, *tD[2] = {}, *loss = nullptr;
   // inference workspace for chunks up to icap rows, fallback list up to fcap cells
   int64_t icap = 0, fcap = 0;
@@ -687,12 +697,12 @@ struct SurrogateState {
   int64_t last_fallback = 0;
 
   void free_train() {
-    for (void *p : {(void *)tX, (void *)tH[0], (void *)tH[1], (void *)tH[2], (void *)tT, (void *)tZ[0],
+    for (void *p : {(void *)tIn, (void *)tX, (void *)tH[0], (void *)tH[1], (void *)tH[2], (void *)tT, (void *)tZ[0],
                     (void *)tZ[1], (void *)tZ[2], (void *)tY, (void *)tG, (void *)tD[0], (void *)tD[1]})
       (void)hipFree(p);
     tX = nullptr;
     tH[0] = tH[1] = tH[2] = nullptr;
-    tT = tY = tG = nullptr;
+    tIn = tT = tY = tG = nullptr;
     tZ[0] = tZ[1] = tZ[2] = nullptr;
     tD[0] = tD[1] = nullptr;
     tcap = 0;
@@ -741,6 +751,7 @@ int ensure_train_ws(SurrogateState *s, int64_t B, hipStream_t st, std::string &e
     SCHK(launch_fill_cols_bf16(s->tH[l], B, kHld, 256, s->aug, st));
     SCHK(dalloc(&s->tZ[l], B * kHld));
   }
+  SCHK(dalloc(&s->tIn, B * (kSurIn + kSurOut)));
   SCHK(dalloc(&s->tT, B * kYld));
   SCHK(dalloc(&s->tY, B * kYld));
   SCHK(hipMemsetAsync(s->tY, 0, (size_t)B * kYld * sizeof(float), st));
@@ -1045,21 +1056,16 @@ static int stage_batch(SurrogateState *s, int64_t B, const float *x, const float
     return 1;
   }
   if (ensure_train_ws(s, B, st, err)) return 1;
-  float *xin = nullptr;
-  SCHK(dalloc(&xin, B * kSurIn));
-  SCHK(hipMemcpyAsync(xin, x, (size_t)B * kSurIn * sizeof(float), hipMemcpyHostToDevice, st));
-  hipLaunchKernelGGL(k_pack_x, dim3(nb256(B)), dim3(256), 0, st, B, (const float *)xin, s->tX);
+  // copies from pageable memory return once the caller's buffer has been read
+  SCHK(hipMemcpyAsync(s->tIn, x, (size_t)B * kSurIn * sizeof(float), hipMemcpyHostToDevice, st));
+  hipLaunchKernelGGL(k_pack_x, dim3(nb256(B)), dim3(256), 0, st, B, (const float *)s->tIn, s->tX);
   SCHK(hipGetLastError());
   if (t) {
-    std::vector<float> tp((size_t)B * kYld, 0.f);
-    for (int64_t r = 0; r < B; ++r)
-      for (int j = 0; j < kSurOut; ++j) tp[(size_t)(r * kYld + j)] = t[r * kSurOut + j];
-    SCHK(hipMemcpyAsync(s->tT, tp.data(), tp.size() * sizeof(float), hipMemcpyHostToDevice, st));
-    SCHK(hipStreamSynchronize(st));
-  } else {
-    SCHK(hipStreamSynchronize(st));
+    float *tin = s->tIn + B * kSurIn;
+    SCHK(hipMemcpyAsync(tin, t, (size_t)B * kSurOut * sizeof(float), hipMemcpyHostToDevice, st));
+    hipLaunchKernelGGL(k_pack_t, dim3(nb256(B * kYld)), dim3(256), 0, st, B, (const float *)tin, s->tT);
+    SCHK(hipGetLastError());
   }
-  SCHK(hipFree(xin));
   return 0;
 }
 
