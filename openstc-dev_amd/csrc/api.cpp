@@ -787,11 +787,11 @@ int build_bc_groups(ostc_solver *s, Block &b) {
 // SourceTerm.cuh:11-37 then the fluxes (SteadySim.cuh:73-78, RK.cuh:109-116):
 // the SST kernel (mu_t, lambda_t, k / omega sources) initialises dq, the
 // chemical source adds to it, the sweeps accumulate.
-int rhs_block(ostc_solver *s, Block &b, bool *dt_done = nullptr) {
+int rhs_block(ostc_solver *s, Block &b, bool *dt_done = nullptr, double *sst_dt = nullptr) {
   bool init = true;
   if (s->n_turb) {
     ostc_solver::Timer t(s, "sst");
-    HIPCHK(launch_sst(b.z, s->P, s->stream));
+    HIPCHK(launch_sst(b.z, s->P, s->stream, sst_dt));
     init = false;
   }
   if (s->P.mix && s->P.reaction == 1 && !s->chem_split) {
@@ -1738,6 +1738,9 @@ int ostc_step_rk3(ostc_solver *s, int nsteps, double *dt_hist, double *res_hist)
   const bool plane = s->P.dim == 2 && s->blocks.size() == 1 && s->blocks[0].mz == 1 && s->blocks[0].inner.empty();
   const bool plane_dt = plane && !fixed && s->n_turb == 0 &&
                         properties_dt_blocks(s->blocks[0].z) <= kMaxDtPartials;
+  // With SST the time step comes out of the k_sst pass of its own stage, under
+  // the same limit, on any lone block.
+  const int sst_blocks = !fixed && s->n_turb && s->blocks.size() == 1 ? sst_dt_blocks(s->blocks[0].z) : 0;
   bool dt_ready = false;  // dt_partial holds the coming stage's time steps
   auto body = [&]() -> int {
     if (fixed) HIPCHK(hipMemcpyAsync(s->w.dt, &fixed_dt, sizeof(double), hipMemcpyHostToDevice, s->stream));
@@ -1752,9 +1755,10 @@ int ostc_step_rk3(ostc_solver *s, int nsteps, double *dt_hist, double *res_hist)
         s->w.dt_copy = d_dt + it * 3 + rk;
         // one block: the k-sweep computes the CFL dt where it can
         bool dt_done = false;
-        const bool fold_dt = !fixed && s->blocks.size() == 1 && !dt_ready;
+        const bool fold_dt = !fixed && s->blocks.size() == 1 && !dt_ready && !sst_blocks;
         for (auto &b : s->blocks)
-          if (rhs_block(s, b, fold_dt ? &dt_done : nullptr)) return 1;
+          if (rhs_block(s, b, fold_dt ? &dt_done : nullptr, sst_blocks ? s->w.dt_partial : nullptr)) return 1;
+        dt_ready = dt_ready || sst_blocks > 0;
         if (fixed)
           HIPCHK(launch_copy_dt(s->w.dt, s->w.dt_copy, s->stream));
         else if (!dt_ready && !dt_done && global_dt_device(s))
@@ -1764,7 +1768,7 @@ int ostc_step_rk3(ostc_solver *s, int nsteps, double *dt_hist, double *res_hist)
           {
             ostc_solver::Timer t(s, "rk_update");
             HIPCHK(launch_rk_update(b.z, s->P, s->d_mech, s->w.dt, rk, s->stream, dt_ready ? s->w.dt_partial : nullptr,
-                                    properties_dt_blocks(b.z), s->w.dt_copy));
+                                    sst_blocks ? sst_blocks : properties_dt_blocks(b.z), s->w.dt_copy));
           }
           if (run_bcs(s, b, true, !ghosts)) return 1;
         }

@@ -181,7 +181,10 @@ hipError_t launch_wall_distance(const ZoneView &z, const double *xyz, const doub
 // mu_t on [-1, m] from the current state (initialisation)
 hipError_t launch_init_mut(const ZoneView &z, const DParams &P, const DMech *m, hipStream_t s);
 // mu_t, lambda_t, the source-Jacobian diagonal, and dq = (0, ..., 0, S_k, S_omega) on the interior
-hipError_t launch_sst(const ZoneView &z, const DParams &P, hipStream_t s);
+// dt_partial (non-null): also dt_local and the smallest time step of each of
+// the sst_dt_blocks workgroups (0: more than kMaxDtPartials)
+hipError_t launch_sst(const ZoneView &z, const DParams &P, hipStream_t s, double *dt_partial = nullptr);
+int sst_dt_blocks(const ZoneView &z);
 // explicit steady step: dq_turb /= 1 - dt J_turb
 hipError_t launch_turb_implicit(const ZoneView &z, const DParams &P, hipStream_t s);
 // smallest singular value of I - dt J per cell (conditioning of the point-implicit step)
