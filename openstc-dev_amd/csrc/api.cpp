@@ -1789,6 +1789,7 @@ int ostc_step_rk3(ostc_solver *s, int nsteps, double *dt_hist, double *res_hist)
     return 0;
   };
   rc = body();
+  s->w.dt_copy = nullptr;
   std::vector<double> hdt(3 * nsteps), hres(5 * nsteps, NAN);
   if (!rc) {
     hipError_t e = hipMemcpyAsync(hdt.data(), d_dt, sizeof(double) * 3 * nsteps, hipMemcpyDeviceToHost, s->stream);

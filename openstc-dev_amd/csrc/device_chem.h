@@ -321,63 +321,6 @@ __device__ inline double d_jacobian_entry(double s, bool on, double ry, double i
   return on ? mw * d_div(s, ry, iry) * 1e+3 : 0.0;
 }
 
-__device__ inline void swap_double(double &a, double &b) {
-  uint2 x = __builtin_bit_cast(uint2, a), y = __builtin_bit_cast(uint2, b);
-  asm volatile("v_swap_b32 %0, %1" : "+v"(x.x), "+v"(y.x));
-  asm volatile("v_swap_b32 %0, %1" : "+v"(x.y), "+v"(y.y));
-  a = __builtin_bit_cast(double, x);
-  b = __builtin_bit_cast(double, y);
-}
-
-// x of A x = b for an N x N system held in registers, b overwritten:
-// elimination with row pivoting, the first largest entry of a column taken
-// (FiniteRateChem.cu:364-418 picks the same rows).  Only what later steps
-// read is swapped; a swap is a branch that a wavefront skips when none of its
-// cells takes that row, and the quotients of a column share the reciprocal of
-// its pivot (d_div rounds them like divisions).
-template <int N>
-__device__ inline void d_gauss_solve(double *A, double *b) {
-  double ip[N];
-#pragma unroll
-  for (int n = 0; n < N; ++n) {
-    int ik = n;
-    double best = fabs(A[n * N + n]);
-#pragma unroll
-    for (int r = n + 1; r < N; ++r) {
-      const double v = fabs(A[r * N + n]);
-      if (v > best) {
-        best = v;
-        ik = r;
-      }
-    }
-    // a register, not the N - n comparisons it came from
-    asm volatile("" : "+v"(ik));
-#pragma unroll
-    for (int r = n + 1; r < N; ++r) {
-      if (r == ik) {
-#pragma unroll
-        for (int c = n; c < N; ++c) swap_double(A[r * N + c], A[n * N + c]);
-        swap_double(b[r], b[n]);
-      }
-    }
-    const double piv = A[n * N + n];
-    ip[n] = 1.0 / piv;
-#pragma unroll
-    for (int r = n + 1; r < N; ++r) {
-      const double f = d_div(A[r * N + n], piv, ip[n]);
-#pragma unroll
-      for (int c = n + 1; c < N; ++c) A[r * N + c] = fma(-f, A[n * N + c], A[r * N + c]);
-      b[r] = fma(-f, b[n], b[r]);
-    }
-  }
-#pragma unroll
-  for (int r = N - 1; r >= 0; --r) {
-#pragma unroll
-    for (int c = r + 1; c < N; ++c) b[r] = fma(-A[r * N + c], b[c], b[r]);
-    b[r] = d_div(b[r], A[r * N + r], ip[r]);
-  }
-}
-
 // FiniteRateChem.cu:364-418 solve_chem_system: Crout-style LU with row
 // pivoting (first maximum wins), then substitution; rhs overwritten.
 template <int N>
