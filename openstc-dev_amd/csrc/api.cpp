@@ -450,7 +450,7 @@ int upload_mech(ostc_solver *s) {
   for (int i = 0; i < ns * ns; ++i) {
     h.WjDivWi_to_One4th[i] = m.WjDivWi_to_One4th[i];
     h.sqrt_WiDivWjPl1Mul8[i] = m.sqrt_WiDivWjPl1Mul8[i];
-    h.binary_diffusivity_coeff[i] = m.binary_diffusivity_coeff[i];
+    h.inv_binary_diffusivity[i] = m.binary_diffusivity_coeff[i] > 0 ? 1 / m.binary_diffusivity_coeff[i] : 0.0;
     h.kb_over_eps_jk[i] = m.kb_over_eps_jk[i];
     h.log_kb_over_eps_jk[i] = m.kb_over_eps_jk[i] > 0 ? std::log(m.kb_over_eps_jk[i]) : 0.0;
   }

@@ -37,7 +37,7 @@ struct DMech {
   double brk[2 * kMS];
   double LJ_potent_inv[kMS], vis_coeff[kMS];
   double WjDivWi_to_One4th[kMS * kMS], sqrt_WiDivWjPl1Mul8[kMS * kMS];
-  double binary_diffusivity_coeff[kMS * kMS], kb_over_eps_jk[kMS * kMS];
+  double inv_binary_diffusivity[kMS * kMS], kb_over_eps_jk[kMS * kMS];  // 1 / D_ab at T = p = 1 and T* = T k_ab
   Reac reac[kMR];
   int stoi_f[kMR * kMS], stoi_b[kMR * kMS];
   // per reaction (rows of n_spec): forward and backward coefficients,
@@ -154,6 +154,14 @@ __device__ inline double d_div(double a, double b, double rb) {
 __device__ inline double d_select(bool c, double a, double b) {
   asm("" : "+v"(a), "+v"(b));
   return c ? a : b;
+}
+
+// 1 / x for finite, normal x within an ulp: the hardware estimate and two
+// Newton-Raphson steps, 5 operations where a division takes 11
+__device__ inline double d_rcp(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = fma(r, fma(-x, r, 1.0), r);
+  return fma(r, fma(-x, r, 1.0), r);
 }
 
 // T and the weights of a0 .. a4 in h / R = a0 T + a1 T^2 / 2 + .. + a4 T^5 / 5 + a5

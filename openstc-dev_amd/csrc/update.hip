@@ -45,7 +45,7 @@ constexpr int kSrcTB = 128;
 constexpr int kMaxEpiReac = 24;  // reactions the point-implicit kernels accept
 
 template <int NS, int NA, int METHOD>
-__global__ void __launch_bounds__(kSrcTB, METHOD == 1 ? 2 : 3) k_source(ZoneView z, const DMech *__restrict__ mech,
+__global__ void __launch_bounds__(kSrcTB, METHOD == 0 ? 3 : 2) k_source(ZoneView z, const DMech *__restrict__ mech,
                                                                        int accumulate) {
   const MechK m = mech_k(mech);
   __shared__ double2 cg[kinetics_slots(NS, METHOD)][kSrcTB];
