@@ -1829,8 +1829,10 @@ static int implicit_block(ostc_solver *s, Block &b) {
   DParams P = s->P;
   if (s->chem_split) P.reaction = 0;
   if (method == 1) {
-    if (!b.walls_inside) return fail("DPLUR: a wall range reaches outside its block");
-    HIPCHK(launch_dplur(b.z, P, s->d_mech, s->prm.get_int("DPLUR_inner_step", 3), b.wall_group, s->stream));
+    // only the inner sweeps zero the wall ranges
+    const int inner = s->prm.get_int("DPLUR_inner_step", 3);
+    if (inner > 0 && !b.walls_inside) return fail("DPLUR: a wall range reaches outside its block");
+    HIPCHK(launch_dplur(b.z, P, s->d_mech, inner, b.wall_group, s->stream));
   } else {
     HIPCHK(launch_chem_implicit(b.z, P, s->stream));
     if (s->n_turb && s->P.turb_implicit == 1) HIPCHK(launch_turb_implicit(b.z, s->P, s->stream));

@@ -119,3 +119,23 @@ def test_c3_steady_inline_chemistry(tmp_path, mech, method):
     assert cells == 8 * 32 * 16 and fb == 0
     s.set_steady_chem(0.0)
     assert s.steady_chem_stats() == (0, 0)
+
+
+def test_wall_range_outside_the_block(tmp_path):
+    """A wall range that reaches one node into the ghosts: the inner sweeps,
+    which zero dq on the wall ranges, are refused; without inner sweeps the
+    range is accepted and a pseudo-iteration matches the oracle."""
+    case = cases.c2_case(24, 16, 12, reconstruction=2, inviscid_scheme=3)
+    for b in case["bcs"]:
+        if b["type"] == 2:
+            raw = list(b["raw"])
+            raw[1] += 1
+            b["raw"] = tuple(raw)
+            break
+    s, z = _air(_steady(case, 1, inner=0, cfl=1.0), tmp_path / "none")
+    s.step_steady(1)
+    z.run_steady(1)
+    _compare(s, z, 1e-12, "c2-dplur-no-sweeps-1")
+    s, _ = _air(_steady(case, 1, inner=3, cfl=1.0), tmp_path / "three")
+    with pytest.raises(ostc.OstcError, match="wall range"):
+        s.step_steady(1)
