@@ -786,12 +786,13 @@ int build_bc_groups(ostc_solver *s, Block &b) {
 
 // SourceTerm.cuh:11-37 then the fluxes (SteadySim.cuh:73-78, RK.cuh:109-116):
 // the SST kernel (mu_t, lambda_t, k / omega sources) initialises dq, the
-// chemical source adds to it, the sweeps accumulate.
-int rhs_block(ostc_solver *s, Block &b, bool *dt_done = nullptr, double *sst_dt = nullptr) {
+// chemical source adds to it, the sweeps accumulate.  sst_dt and flat as
+// launch_sst takes them.
+int rhs_block(ostc_solver *s, Block &b, bool *dt_done = nullptr, double *sst_dt = nullptr, bool flat = false) {
   bool init = true;
   if (s->n_turb) {
     ostc_solver::Timer t(s, "sst");
-    HIPCHK(launch_sst(b.z, s->P, s->stream, sst_dt));
+    HIPCHK(launch_sst(b.z, s->P, s->stream, sst_dt, flat));
     init = false;
   }
   if (s->P.mix && s->P.reaction == 1 && !s->chem_split) {
@@ -1757,7 +1758,9 @@ int ostc_step_rk3(ostc_solver *s, int nsteps, double *dt_hist, double *res_hist)
         bool dt_done = false;
         const bool fold_dt = !fixed && s->blocks.size() == 1 && !dt_ready && !sst_blocks;
         for (auto &b : s->blocks)
-          if (rhs_block(s, b, fold_dt ? &dt_done : nullptr, sst_blocks ? s->w.dt_partial : nullptr)) return 1;
+          if (rhs_block(s, b, fold_dt ? &dt_done : nullptr, sst_blocks ? s->w.dt_partial : nullptr,
+                        plane && it + rk > 0))
+            return 1;
         dt_ready = dt_ready || sst_blocks > 0;
         if (fixed)
           HIPCHK(launch_copy_dt(s->w.dt, s->w.dt_copy, s->stream));

@@ -182,8 +182,10 @@ hipError_t launch_wall_distance(const ZoneView &z, const double *xyz, const doub
 hipError_t launch_init_mut(const ZoneView &z, const DParams &P, const DMech *m, hipStream_t s);
 // mu_t, lambda_t, the source-Jacobian diagonal, and dq = (0, ..., 0, S_k, S_omega) on the interior
 // dt_partial (non-null): also dt_local and the smallest time step of each of
-// the sst_dt_blocks workgroups (0: more than kMaxDtPartials)
-hipError_t launch_sst(const ZoneView &z, const DParams &P, hipStream_t s, double *dt_partial = nullptr);
+// the sst_dt_blocks workgroups (0: more than kMaxDtPartials); flat: a 2-D
+// block whose k-ghost planes are not up to date and stand for copies of k = 0
+hipError_t launch_sst(const ZoneView &z, const DParams &P, hipStream_t s, double *dt_partial = nullptr,
+                      bool flat = false);
 int sst_dt_blocks(const ZoneView &z);
 // explicit steady step: dq_turb /= 1 - dt J_turb
 hipError_t launch_turb_implicit(const ZoneView &z, const DParams &P, hipStream_t s);

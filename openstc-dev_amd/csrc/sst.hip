@@ -47,11 +47,12 @@ __global__ void __launch_bounds__(kTB) k_wall_distance(ZoneView z, const double 
   if (live) z.wdist[p] = sqrt(d2);
 }
 
-// central point gradient 0.5 (xi_c dF/di + eta_c dF/dj + zeta_c dF/dk)
-__device__ inline void point_grad(const ZoneView &z, const double *f, int64_t p, const double *mm, double *g) {
-  // in 2-D the k-ghost planes are copies of k = 0, refreshed at the end of a run
+// central point gradient 0.5 (xi_c dF/di + eta_c dF/dj + zeta_c dF/dk); flat:
+// k planes that are copies of each other and not up to date in memory
+__device__ inline void point_grad(const ZoneView &z, const double *f, int64_t p, const double *mm, bool flat,
+                                  double *g) {
   const double di = f[p + 1] - f[p - 1], dj = f[p + z.d2] - f[p - z.d2];
-  const double dk = z.mz > 1 ? f[p + z.d1] - f[p - z.d1] : 0.0;
+  const double dk = flat ? 0.0 : f[p + z.d1] - f[p - z.d1];
 #pragma unroll
   for (int c = 0; c < 3; ++c) g[c] = 0.5 * (mm[c] * di + mm[3 + c] * dj + mm[6 + c] * dk);
 }
@@ -65,9 +66,9 @@ __device__ inline void load_metric(const ZoneView &z, int64_t p, double *mm) {
 __device__ inline double sst_mut(const ZoneView &z, int ns, int64_t p, double mul) {
   double mm[9], gu[3], gv[3], gw[3];
   load_metric(z, p, mm);
-  point_grad(z, z.bv + z.sz, p, mm, gu);
-  point_grad(z, z.bv + 2 * z.sz, p, mm, gv);
-  point_grad(z, z.bv + 3 * z.sz, p, mm, gw);
+  point_grad(z, z.bv + z.sz, p, mm, false, gu);
+  point_grad(z, z.bv + 2 * z.sz, p, mm, false, gv);
+  point_grad(z, z.bv + 3 * z.sz, p, mm, false, gw);
   const double rho = z.bv[p], tke = z.sv[(int64_t)ns * z.sz + p], omega = z.sv[(int64_t)(ns + 1) * z.sz + p];
   const double vort = sqrt((gv[0] - gu[1]) * (gv[0] - gu[1]) + (gw[0] - gu[2]) * (gw[0] - gu[2]) +
                            (gw[1] - gv[2]) * (gw[1] - gv[2]));
@@ -131,15 +132,15 @@ __device__ inline double zeman_correction(double mt, double gamma_p1) {
 // Jacobian diagonal (-2 beta* omega, -2 beta omega).  dq is initialised here:
 // zero on the flow and species rows, the source on the k and omega rows.
 template <int NS>
-__device__ inline void sst_cell(const ZoneView &z, const DParams &P, int64_t p, int64_t q) {
+__device__ inline void sst_cell(const ZoneView &z, const DParams &P, int64_t p, int64_t q, bool flat) {
   const double *ks = z.sv + (int64_t)NS * z.sz, *ws = z.sv + (int64_t)(NS + 1) * z.sz;
   double mm[9], gu[3], gv[3], gw[3], gk[3], go[3];
   load_metric(z, p, mm);
-  point_grad(z, z.bv + z.sz, p, mm, gu);
-  point_grad(z, z.bv + 2 * z.sz, p, mm, gv);
-  point_grad(z, z.bv + 3 * z.sz, p, mm, gw);
-  point_grad(z, ks, p, mm, gk);
-  point_grad(z, ws, p, mm, go);
+  point_grad(z, z.bv + z.sz, p, mm, flat, gu);
+  point_grad(z, z.bv + 2 * z.sz, p, mm, flat, gv);
+  point_grad(z, z.bv + 3 * z.sz, p, mm, flat, gw);
+  point_grad(z, ks, p, mm, flat, gk);
+  point_grad(z, ws, p, mm, flat, go);
   const double u_x = gu[0], u_y = gu[1], u_z = gu[2], v_x = gv[0], v_y = gv[1], v_z = gv[2];
   const double w_x = gw[0], w_y = gw[1], w_z = gw[2];
   const double rho = z.bv[p], tke = ks[p], omega = ws[p];
@@ -207,7 +208,7 @@ __device__ inline void sst_cell(const ZoneView &z, const DParams &P, int64_t p, 
 // workgroup in dt_partial, which the update reduces -- two launches of 4 and
 // 2 us less per stage, a tenth of a small block's.
 template <int NS>
-__global__ void __launch_bounds__(kTB) k_sst(ZoneView z, DParams P, double *dt_partial) {
+__global__ void __launch_bounds__(kTB) k_sst(ZoneView z, DParams P, double *dt_partial, int flat) {
   const int64_t t = (int64_t)blockIdx.x * kTB + threadIdx.x;
   const int64_t n = (int64_t)z.mx * z.my * z.mz;
   double best = 1e+6;
@@ -215,7 +216,7 @@ __global__ void __launch_bounds__(kTB) k_sst(ZoneView z, DParams P, double *dt_p
     int i, j, k;
     unflatten3(t, z.mx, z.my, i, j, k);
     const int64_t p = z.at(i, j, k), q = z.at0(i, j, k);
-    sst_cell<NS>(z, P, p, q);
+    sst_cell<NS>(z, P, p, q, flat != 0);
     if (dt_partial) {
       const double dtl = cell_dt<(NS > 0)>(z, P, p, q);
       z.dt_local[q] = dtl;
@@ -268,12 +269,13 @@ int sst_dt_blocks(const ZoneView &z) {
   return n <= kMaxDtPartials ? (int)n : 0;
 }
 
-hipError_t launch_sst(const ZoneView &z, const DParams &P, hipStream_t s, double *dt_partial) {
+hipError_t launch_sst(const ZoneView &z, const DParams &P, hipStream_t s, double *dt_partial, bool flat) {
   if (!z.mut || !z.tcond || !z.wdist || P.nt != 2 || (P.turb_implicit == 1 && !z.turb_jac))
     return hipErrorInvalidValue;
   const int64_t n = (int64_t)z.mx * z.my * z.mz;
   return with_species(P.ns, [&](auto c) {
-    hipLaunchKernelGGL(k_sst<decltype(c)::value>, dim3(nblk(n, kTB)), dim3(kTB), 0, s, z, P, dt_partial);
+    hipLaunchKernelGGL(k_sst<decltype(c)::value>, dim3(nblk(n, kTB)), dim3(kTB), 0, s, z, P, dt_partial,
+                       flat ? 1 : 0);
     return hipGetLastError();
   });
 }

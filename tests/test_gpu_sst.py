@@ -73,6 +73,30 @@ def test_plate_init_and_rhs(tmp_path):
     assert abs(dt_p - dt_o) / dt_o < 1e-14
 
 
+def test_rhs_reads_the_uploaded_k_planes(tmp_path):
+    """k planes that are no copies of k = 0: the source's k differences come
+    from memory, as in the oracle.  The ghost planes next to k = 0 get their
+    own velocities, k and omega."""
+    case, s, z = _plate(tmp_path)
+    shape = cases.ghost_shape(case["mx"], case["my"], case["mz"], case["ngg"])
+    rng = np.random.default_rng(3)
+    for f, rows in (("bv", (1, 2, 3)), ("sv", (0, 1))):
+        a = s.download(f).reshape((-1,) + shape)
+        for r in rows:
+            for k in (case["ngg"] - 1, case["ngg"] + 1):
+                a[r, k] *= 1 + 0.1 * rng.random(shape[1:])
+                if r == 3:
+                    a[r, k] += 10.0 * rng.random(shape[1:])
+        s.upload(f, a)
+        z.field(f)[:] = a.ravel()
+    s.rhs()
+    z.rhs()
+    dq_p, dq_o = s.download("dq").reshape(7, -1), z.field("dq").reshape(7, -1)
+    errs = dict(k=relerr(dq_p[5], dq_o[5]), omega=relerr(dq_p[6], dq_o[6]), mut=relerr(s.download("mut"), z.field("mut")))
+    print("plate rhs, own k planes", {k: "%.2e" % v for k, v in errs.items()}, flush=True)
+    assert max(errs.values()) < 1e-12, errs
+
+
 def test_plate_rk3(tmp_path):
     case, s, z = _plate(tmp_path)
     s.step(1)
