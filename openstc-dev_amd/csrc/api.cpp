@@ -68,6 +68,7 @@ struct Block {
   std::vector<BCGroup> bc_plane;    // 2-D: their k = 0 points only
   BCGroup wall_group;               // the wall ranges, for DPLUR
   bool walls_inside = true;         // every wall range lies inside the block (DPLUR needs it)
+  bool farfield = false;            // some range is a farfield
   ZoneView z{};
   std::vector<void *> mem;
 };
@@ -730,6 +731,7 @@ int build_bc_groups(ostc_solver *s, Block &b) {
     }
     if (empty) continue;
     live.push_back(c);
+    b.farfield = b.farfield || c.type == BC_FARFIELD;
     if (c.type == BC_WALL) {
       walls.push_back(c);
       b.walls_inside = b.walls_inside && inside;
@@ -1776,12 +1778,15 @@ int ostc_step_rk3(ostc_solver *s, int nsteps, double *dt_hist, double *res_hist)
           if (run_bcs(s, b, true, !ghosts)) return 1;
         }
         if (exchange_all(s, true)) return 1;
-        // the last stage's boundary ranges read the planes that the stage before left
+        // The last stage's boundary ranges read the planes that the stage
+        // before left: the state near the faces, and a mixture farfield gamma.
         if (s->P.dim == 2 && (ghosts || to_go == 1))
           for (auto &b : s->blocks) HIPCHK(launch_eliminate_k(b.z, s->P, true, s->stream, !ghosts));
         dt_ready = plane_dt && to_go > 0;
         for (auto &b : s->blocks)
-          if (properties_block(s, b, true, ghosts, dt_ready ? s->w.dt_partial : nullptr, to_go == 1)) return 1;
+          if (properties_block(s, b, true, ghosts || (to_go == 1 && s->P.mix && b.farfield),
+                               dt_ready ? s->w.dt_partial : nullptr, to_go == 1))
+            return 1;
       }
       if (step % os == 0 || step == 1) {
         ostc_solver::Timer t(s, "residual");

@@ -9,15 +9,39 @@ from ostc import cases
 
 pytestmark = pytest.mark.gpu
 
-FIELDS = ("bv", "sv", "cv", "dq", "acoustic", "mul", "cond", "dt_local")
+# vel and mach on the ghost planes are what the boundary ranges derive there
+# from the planes that a stage before left
+FIELDS = ("bv", "sv", "cv", "dq", "vel", "mach", "acoustic", "mul", "cond", "gamma", "cp", "rhoD", "mut", "turb_cond",
+          "dt_local")
+
+
+def _case(kind, size):
+    if kind in ("mixing", "farfield"):
+        case = cases.c3_case(*size)
+        if kind == "farfield":
+            case["setup"]["array string boundary_conditions"] = ["air_stream", "fuel_stream", "outflow", "farfield"]
+            case["setup"]["struct farfield"] = [
+                ("string", "type", "farfield"), ("int", "label", 4), ("real", "mach", 2.0),
+                ("real", "pressure", 101325.0), ("real", "temperature", 1500.0), ("real", "u", 1.0),
+                ("real", "v", 0.0), ("real", "w", 0.0), ("real", "O2", 0.233), ("real", "N2", 0.767)]
+            for b in case["bcs"]:
+                if b["type"] == 3:
+                    b["type"], b["label"] = 4, 4
+        return case
+    if kind == "plate":
+        return cases.sst_plate_case(*size)
+    case = cases.c1_case(*size)
+    if kind == "fixed":
+        case["setup"]["bool fixed_time_step"], case["setup"]["real dt"] = 1, 2e-7
+    return case
 
 
 def _solver(kind, size, root):
-    case = {"air": cases.c1_case, "mixing": cases.c3_case, "plate": cases.sst_plate_case}[kind](*size)
-    if kind == "air":
+    case = _case(kind, size)
+    if case["name"] == "c1":
         return case, ostc.solver_for_case(case, root)
     s = ostc.solver_for_case(case, root, initial=False)
-    if kind == "mixing":
+    if case["name"] == "c3":
         st = {}
         for k in ("air_stream", "fuel_stream"):
             o = s.inflow_state(k, 16)
@@ -33,7 +57,8 @@ def _solver(kind, size, root):
 
 # 14 x 14 points with ghosts are less than one workgroup, 513 x 511 need more
 # than the 1024 partial minima that the update reduces itself
-@pytest.mark.parametrize("kind,size", [("air", (12, 12)), ("air", (62, 37)), ("air", (513, 511)), ("mixing", (33, 17)),
+@pytest.mark.parametrize("kind,size", [("air", (12, 12)), ("air", (62, 37)), ("air", (513, 511)), ("fixed", (62, 37)),
+                                       ("mixing", (33, 17)), ("farfield", (33, 17)),
                                        ("plate", (60, 40))])
 def test_calls_cut_differently(tmp_path, kind, size):
     out = []
