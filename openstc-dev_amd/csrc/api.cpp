@@ -68,6 +68,7 @@ struct Block {
   std::vector<BCGroup> bc_plane;    // 2-D: their k = 0 points only
   BCGroup wall_group;               // the wall ranges, for DPLUR
   bool walls_inside = true;         // every wall range lies inside the block (DPLUR needs it)
+  bool on_edges = true;             // every range's face is the first or last layer of its direction
   bool farfield = false;            // some range is a farfield
   ZoneView z{};
   std::vector<void *> mem;
@@ -731,6 +732,7 @@ int build_bc_groups(ostc_solver *s, Block &b) {
     }
     if (empty) continue;
     live.push_back(c);
+    b.on_edges = b.on_edges && c.rs[c.face] == (c.dir < 0 ? 0 : m[c.face] - 1);
     b.farfield = b.farfield || c.type == BC_FARFIELD;
     if (c.type == BC_WALL) {
       walls.push_back(c);
@@ -1779,9 +1781,10 @@ int ostc_step_rk3(ostc_solver *s, int nsteps, double *dt_hist, double *res_hist)
         }
         if (exchange_all(s, true)) return 1;
         // The last stage's boundary ranges read the planes that the stage
-        // before left: the state near the faces, and a mixture farfield gamma.
+        // before left: the state near the faces (everywhere for a face that
+        // is not an edge of the block), and a mixture farfield gamma.
         if (s->P.dim == 2 && (ghosts || to_go == 1))
-          for (auto &b : s->blocks) HIPCHK(launch_eliminate_k(b.z, s->P, true, s->stream, !ghosts));
+          for (auto &b : s->blocks) HIPCHK(launch_eliminate_k(b.z, s->P, true, s->stream, !ghosts && b.on_edges));
         dt_ready = plane_dt && to_go > 0;
         for (auto &b : s->blocks)
           if (properties_block(s, b, true, ghosts || (to_go == 1 && s->P.mix && b.farfield),

@@ -33,6 +33,8 @@ def _case(kind, size):
     case = cases.c1_case(*size)
     if kind == "fixed":
         case["setup"]["bool fixed_time_step"], case["setup"]["real dt"] = 1, 2e-7
+    if kind == "inside":  # a symmetry patch on a layer inside the block
+        case["bcs"].append(dict(type=3, raw=(30, 30, 8, 20, 0, 0), label=3))
     return case
 
 
@@ -58,7 +60,7 @@ def _solver(kind, size, root):
 # 14 x 14 points with ghosts are less than one workgroup, 513 x 511 need more
 # than the 1024 partial minima that the update reduces itself
 @pytest.mark.parametrize("kind,size", [("air", (12, 12)), ("air", (62, 37)), ("air", (513, 511)), ("fixed", (62, 37)),
-                                       ("mixing", (33, 17)), ("farfield", (33, 17)),
+                                       ("inside", (62, 37)), ("mixing", (33, 17)), ("farfield", (33, 17)),
                                        ("plate", (60, 40))])
 def test_calls_cut_differently(tmp_path, kind, size):
     out = []
