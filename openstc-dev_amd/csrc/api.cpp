@@ -1740,8 +1740,13 @@ int ostc_step_rk3(ostc_solver *s, int nsteps, double *dt_hist, double *res_hist)
   // the last stage alone.  Its properties pass also gives the next stage's
   // time step (not with SST, whose mu_t of that stage enters it), when the
   // update's workgroups can each reduce the partial minima (kMaxDtPartials).
-  const bool plane = s->P.dim == 2 && s->blocks.size() == 1 && s->blocks[0].mz == 1 && s->blocks[0].inner.empty();
-  const bool plane_dt = plane && !fixed && s->n_turb == 0 &&
+  // Not with a farfield: it stores |u| only where the flow is not leaving
+  // faster than sound, with a mixture's gamma of its own k plane (zero on the
+  // outer ones, which have no properties), so what stands on the ghost planes
+  // is from the last stage that stored it.
+  const bool lone = s->P.dim == 2 && s->blocks.size() == 1 && s->blocks[0].mz == 1 && s->blocks[0].inner.empty();
+  const bool plane = lone && !s->blocks[0].farfield;
+  const bool plane_dt = lone && !fixed && s->n_turb == 0 &&
                         properties_dt_blocks(s->blocks[0].z) <= kMaxDtPartials;
   // With SST the time step comes out of the k_sst pass of its own stage, under
   // the same limit, on any lone block.
@@ -1782,14 +1787,12 @@ int ostc_step_rk3(ostc_solver *s, int nsteps, double *dt_hist, double *res_hist)
         if (exchange_all(s, true)) return 1;
         // The last stage's boundary ranges read the planes that the stage
         // before left: the state near the faces (everywhere for a face that
-        // is not an edge of the block), and a mixture farfield gamma.
+        // is not an edge of the block).
         if (s->P.dim == 2 && (ghosts || to_go == 1))
           for (auto &b : s->blocks) HIPCHK(launch_eliminate_k(b.z, s->P, true, s->stream, !ghosts && b.on_edges));
         dt_ready = plane_dt && to_go > 0;
         for (auto &b : s->blocks)
-          if (properties_block(s, b, true, ghosts || (to_go == 1 && s->P.mix && b.farfield),
-                               dt_ready ? s->w.dt_partial : nullptr, to_go == 1))
-            return 1;
+          if (properties_block(s, b, true, ghosts, dt_ready ? s->w.dt_partial : nullptr, to_go == 1)) return 1;
       }
       if (step % os == 0 || step == 1) {
         ostc_solver::Timer t(s, "residual");
