@@ -11,11 +11,13 @@ from helpers import BV_GROUPS, grouped, oracle_zone
 pytestmark = pytest.mark.gpu
 
 EXTRA = {
-    # an outflow patch under the wall: the later wall overwrites it
+    # an outflow patch on the lower symmetry face: outflow ranges go first, the
+    # symmetry then overwrites what both write
     "overlap": [dict(type=6, raw=(5, 12, 0, 0, 0, 0), label=6)],
-    # two wall patches over the same nodes, and one that shares an end node
-    "shared": [dict(type=2, raw=(8, 20, 0, 0, 0, 0), label=2, t_wall=300.0, isothermal=True),
-               dict(type=2, raw=(20, 33, 0, 0, 0, 0), label=2, t_wall=300.0, isothermal=True)],
+    # a cold and a hot wall on the lower face, in this order, that share nodes
+    # 14 to 20: the hot one has the last word there
+    "shared": [dict(type=2, raw=(8, 20, 0, 0, 0, 0), label=20, t_wall=250.0, isothermal=True),
+               dict(type=2, raw=(14, 33, 0, 0, 0, 0), label=21, t_wall=900.0, isothermal=True)],
     # a patch whose ghosts and interior reach into another's corner
     "corner": [dict(type=6, raw=(39, 39, 0, 6, 0, 0), label=6), dict(type=6, raw=(37, 39, 0, 0, 0, 0), label=6)],
 }
@@ -24,11 +26,13 @@ EXTRA = {
 @pytest.mark.parametrize("extra", sorted(EXTRA))
 def test_ranges_that_meet(tmp_path, extra):
     case = cases.c1_case(40, 20)
-    for b in case["bcs"]:
-        if b["type"] == 2:
-            for e in EXTRA[extra]:
-                if e["type"] == 2:
-                    e.update(t_wall=b.get("t_wall", 300.0), label=b["label"])
+    walls = [b for b in EXTRA[extra] if b["type"] == 2]
+    for b in walls:
+        name = "wall%d" % b["label"]
+        case["setup"]["array string boundary_conditions"].append(name)
+        case["setup"]["struct " + name] = [("string", "type", "wall"), ("int", "label", b["label"]),
+                                           ("string", "thermal_type", "isothermal"),
+                                           ("real", "temperature", b["t_wall"])]
     case["bcs"] = case["bcs"] + EXTRA[extra]
     s = ostc.solver_for_case(case, str(tmp_path / extra))
     z = oracle_zone(case)
@@ -37,3 +41,7 @@ def test_ranges_that_meet(tmp_path, extra):
     errs = grouped(s.download("bv"), z.field("bv"), 6, BV_GROUPS)
     print(extra, {k: "%.1e" % v for k, v in errs.items()}, flush=True)
     assert max(errs.values()) < 1e-12 and np.all(np.isfinite(s.download("bv")))
+    if walls:
+        t = s.download("bv").reshape((6,) + cases.ghost_shape(case["mx"], case["my"], case["mz"], case["ngg"]))[5]
+        g = case["ngg"]
+        assert t[g, g, g + 10] == 250.0 and t[g, g, g + 17] == 900.0
