@@ -11,7 +11,7 @@
 // Tile: 64 x 64 outputs per workgroup of 4 wavefronts (each 32 x 32 = 2 x 2
 // MFMA tiles), K step 64, the next step's operands loaded into registers
 // while the current one is multiplied.  The products of a mini-batch are
-// short (K = 24 to 264 forward, one 300-row share of the batch backward), so
+// short (K = 24 to 264 forward, shares of 256 or 384 of 8,192 rows backward), so
 // a tile's time is a few global-load latencies: K steps of 32 that waited for
 // their own loads, with LDS moved in 2-byte pieces, took 13 / 17 / 20 us for
 // the forward, input-gradient and weight-gradient products of 8,192 rows;
@@ -207,6 +207,10 @@ hipError_t launch_gemm(const GemmArgs &g, const void *A, bool a_bf16, const void
   if (((uintptr_t)A | (uintptr_t)B) % 16) return hipErrorInvalidValue;
   if (split_k < 1) split_k = 1;
   if (split_k > 1 && g.mode != EPI_ATOMIC) return hipErrorInvalidValue;
+  // shares are whole K steps (k_gemm), so fewer than asked for may cover K; an
+  // empty one would only add zeros to every output
+  const int share = ((g.K + split_k - 1) / split_k + BK - 1) / BK * BK;
+  split_k = (g.K + share - 1) / share;
   const dim3 grid((g.N + BN - 1) / BN, (g.M + BM - 1) / BM, split_k), blk(256);
   if (a_bf16 && b_bf16)
     hipLaunchKernelGGL((k_gemm<__bf16, __bf16>), grid, blk, 0, s, g, (const __bf16 *)A, (const __bf16 *)B);

@@ -22,9 +22,10 @@ def solver(tmp_path_factory):
     return s
 
 
-# 8: one 8-row step; 56, 72: below and above a tile of 64; 264: above a
-# weight-gradient share of 256; 1000: several shares, the last one partial
-@pytest.mark.parametrize("batch", [8, 56, 72, 264, 1000])
+# 8: one 8-row step; 56, 72: below and above a tile of 64; 264: a fifth K step
+# of 8 rows in the one share; 1000: three shares, the last one partial; 8192:
+# the 25 shares asked for are 21 of 384 rows and one of 128
+@pytest.mark.parametrize("batch", [8, 56, 72, 264, 1000, 8192])
 def test_gradient_batch_sizes(solver, batch):
     rng = np.random.default_rng(batch)
     p = mo.pack([(W, 0.1 * rng.standard_normal(b.shape)) for W, b in mo.unpack(mo.init_params(8))]).astype(np.float32)
