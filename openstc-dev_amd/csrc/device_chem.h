@@ -132,8 +132,8 @@ __device__ inline void d_chem_rates(MechK m, double rho, double t, const double 
   for (int l = 0; l < NS; ++l) omega[l] = creation[l] * (m->mw[l] * 1e+3) - destr[l] * (m->mw[l] * 1e+3);
 }
 
-// The EPI Jacobian J from the parked rates of progress; with EPI, A = I - dt J
-template <int NS, bool EPI = true>
+// A = I - dt J with the EPI Jacobian J from the parked rates of progress
+template <int NS>
 __device__ inline void d_epi_matrix(MechK m, double rho, const double *Y, double dt,
                                     const double *q, int stride, double *A) {
 #pragma unroll
@@ -154,7 +154,7 @@ __device__ inline void d_epi_matrix(MechK m, double rho, const double *Y, double
 #pragma unroll
     for (int a = 0; a < NS; ++a) {
       const double J = on ? m->mw[a] * (A[a * NS + n] / (rho * Y[n])) * 1e+3 : 0.0;
-      A[a * NS + n] = EPI ? (a == n ? 1.0 : 0.0) - dt * J : J;
+      A[a * NS + n] = (a == n ? 1.0 : 0.0) - dt * J;
     }
   }
 }
@@ -398,10 +398,10 @@ __device__ inline void species_viscosities(MechK m, double t, double *vis, doubl
 #pragma unroll
   for (int l = 0; l < NS; ++l) {
     const double x5 = t * m->LJ_potent_inv[l] + 0.5;
-    const double ci = 1.147 * exp(-0.145 * (lt + m->log_LJ_potent_inv[l])) + d_rcp(x5 * x5);
-    vis[l] = m->vis_coeff[l] * st * d_rcp(ci);
+    const double ci = 1.147 * exp(-0.145 * (lt + m->log_LJ_potent_inv[l])) + rcp(x5 * x5);
+    vis[l] = m->vis_coeff[l] * st * rcp(ci);
     sv[l] = sqrt(vis[l]);
-    isv[l] = d_rcp(sv[l]);
+    isv[l] = rcp(sv[l]);
   }
 }
 
@@ -433,7 +433,7 @@ __device__ inline double d_viscosity(MechK m, double t, double mw_total, const d
 
 // Transport.cu:40-110 compute_transport_property.  The 36 pairs' collision
 // integrals and diffusivities, the 9 species' viscosities and Wilke's sums
-// would be 136 divisions; they are reciprocals within an ulp (d_rcp) and one
+// would be 136 divisions; they are reciprocals within an ulp (rcp) and one
 // division (k_properties<9>: 512x256 cells 38 -> 32 us, 1.18 M cells 191 -> 166).
 template <int NS>
 __device__ inline void d_transport(MechK m, double t, double p, double rho, const double *Y,
@@ -461,9 +461,9 @@ __device__ inline void d_transport(MechK m, double t, double p, double rho, cons
       vt += pf * X[b];
     }
     const double ct = 1.065 * vt - 0.065 * X[a];
-    viscosity += vis[a] * X[a] * d_rcp(vt);
+    viscosity += vis[a] * X[a] * rcp(vt);
     const double la = vis[a] * (cp[a] + 1.25 * kRuD * m->mw_inv[a]);
-    conductivity += la * X[a] * d_rcp(ct);
+    conductivity += la * X[a] * rcp(ct);
   }
   mu = viscosity;
   lam = conductivity;
@@ -476,7 +476,7 @@ __device__ inline void d_transport(MechK m, double t, double p, double rho, cons
 #pragma unroll
     for (int b = a + 1; b < NS; ++b) {
       const double tr = t * m->kb_over_eps_jk[a * NS + b];
-      const double od = exp(-0.145 * (lt + m->log_kb_over_eps_jk[a * NS + b])) + d_rcp((tr + 0.5) * (tr + 0.5));
+      const double od = exp(-0.145 * (lt + m->log_kb_over_eps_jk[a * NS + b])) + rcp((tr + 0.5) * (tr + 0.5));
       idij[a * NS - a * (a + 1) / 2 + (b - a - 1)] = od * (m->inv_binary_diffusivity[a * NS + b] * it32p);
     }
 #pragma unroll
@@ -490,7 +490,7 @@ __device__ inline void d_transport(MechK m, double t, double p, double rho, cons
         den += (X[n] + 1e-12) * idij[a * NS - a * (a + 1) / 2 + (b - a - 1)];
       }
     }
-    rhoD[l] = rho * num * mwi * d_rcp(den);
+    rhoD[l] = rho * num * mwi * rcp(den);
   }
 }
 

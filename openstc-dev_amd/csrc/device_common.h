@@ -156,13 +156,19 @@ __device__ inline double d_select(bool c, double a, double b) {
   return c ? a : b;
 }
 
-// 1 / x for finite, normal x within an ulp: the hardware estimate and two
-// Newton-Raphson steps, 5 operations where a division takes 11
-__device__ inline double d_rcp(double x) {
+// 1 / x for finite, normal x: the hardware estimate refined by two
+// Newton-Raphson steps r <- r + r (1 - x r), each squaring the relative
+// error, so the result is within an ulp of 1 / x, in 5 operations where a
+// division takes 11.  A quotient a * rcp(b) then differs from a / b by rounding
+// only; shared denominators are inverted once.
+__device__ inline double rcp(double x) {
   double r = __builtin_amdgcn_rcp(x);
-  r = fma(r, fma(-x, r, 1.0), r);
-  return fma(r, fma(-x, r, 1.0), r);
+  double e = fma(-x, r, 1.0);
+  r = fma(r, e, r);
+  e = fma(-x, r, 1.0);
+  return fma(r, e, r);
 }
+__device__ inline float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 
 // T and the weights of a0 .. a4 in h / R = a0 T + a1 T^2 / 2 + .. + a4 T^5 / 5 + a5
 struct TPow {

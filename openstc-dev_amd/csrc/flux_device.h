@@ -112,21 +112,6 @@ __device__ inline void recon_pv(const ZoneView &z, int recon, MechK m, int64_t p
   }
 }
 
-// ------------------------------------------------------ reciprocals
-// 1/x for finite, normal x: the hardware estimate refined by two
-// Newton-Raphson steps r <- r + r (1 - x r), each squaring the relative
-// error, so the result is within an ulp of 1/x.  A quotient a * rcp(b)
-// then differs from a / b by rounding only; shared denominators are
-// inverted once.
-__device__ inline double rcp(double x) {
-  double r = __builtin_amdgcn_rcp(x);
-  double e = fma(-x, r, 1.0);
-  r = fma(r, e, r);
-  e = fma(-x, r, 1.0);
-  return fma(r, e, r);
-}
-__device__ inline float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
-
 // ------------------------------------------------------ AWENO (air)
 // AWENO.cu:151-206 WENO5 on the six characteristic values v[s] of the
 // stencil points s = 0..5 (i-2..i+3): v-(i+1/2) and v+(i+1/2).
@@ -433,24 +418,6 @@ __device__ inline void mix_roe_state(MechK m, const R *cl, const R *cr, const R 
   E.U = E.nx * E.u + E.ny * E.v + E.nz * E.w;
 }
 
-// characteristic amplitudes w = L Q of a conservative vector Q
-template <int NS, int NT, typename R>
-__device__ inline void mix_left(const MixEig<NS, NT, R> &E, const R *Q, R *wv) {
-  constexpr int NV = 5 + NS + NT;
-  R c1 = E.gm1 * (E.ek * Q[0] - E.u * Q[1] - E.v * Q[2] - E.w * Q[3] + Q[4]) * rcp(E.c2);
-#pragma unroll
-  for (int l = 0; l < NS; ++l) c1 += E.a[l] * Q[5 + l];
-  const R c2v = (E.nx * Q[1] + E.ny * Q[2] + E.nz * Q[3] - E.U * Q[0]) * E.ic;
-  const R c3 = Q[0] - c1;
-  wv[0] = R(0.5) * (c1 - c2v);
-  wv[1] = E.nx * c3 - ((E.nz * E.v - E.ny * E.w) * Q[0] - E.nz * Q[2] + E.ny * Q[3]) * E.ic;
-  wv[2] = E.ny * c3 - ((E.nx * E.w - E.nz * E.u) * Q[0] - E.nx * Q[3] + E.nz * Q[1]) * E.ic;
-  wv[3] = E.nz * c3 - ((E.ny * E.u - E.nx * E.v) * Q[0] - E.ny * Q[1] + E.nx * Q[2]) * E.ic;
-  wv[4] = R(0.5) * (c1 + c2v);
-#pragma unroll
-  for (int l = 5; l < NV; ++l) wv[l] = Q[l] - E.y[l - 5] * Q[0];
-}
-
 // conservative vector Q = R w of characteristic amplitudes w
 template <int NS, int NT, typename R>
 __device__ inline void mix_right(const MixEig<NS, NT, R> &E, const R *wv, R *Q) {
@@ -550,8 +517,7 @@ __device__ inline bool mix_side_ok(const R *pv) {
 // Register use: the scalar waves Q_{5+l} - Y~_l Q_0 are formed and
 // interpolated one scalar at a time (their stencil is read when needed), and
 // the acoustic rows keep only the 6 x 5 flow rows of the stencil, so the
-// 6 x NV amplitude block of the whole stencil is never live at once; the
-// arithmetic and its order are those of mix_left / weno5 per component.
+// 6 x NV amplitude block of the whole stencil is never live at once.
 template <int NS, int NT, typename R>
 __device__ inline void aweno_mix(const ZoneView &z, MechK m, int64_t p0, int64_t st,
                                  const R *mk0, const R *mk1, R *pl, R *pr) {

@@ -42,7 +42,7 @@ __device__ inline double wave_sum(double v) {
 // and 19 reactions: 127 -> 41 us; 20,503 cells: 63 -> 33 us; with the Jacobian,
 // 1.18 M cells: 1.37 -> 0.55 ms (0.9 GB of it, the Jacobian's stores).
 constexpr int kSrcTB = 128;
-constexpr int kMaxEpiReac = 24;  // reactions the point-implicit kernels accept
+constexpr int kMaxEpiReac = 24;  // reactions that the point-implicit paths accept (the batch parks their rates in LDS)
 
 template <int NS, int NA, int METHOD>
 __global__ void __launch_bounds__(kSrcTB, METHOD == 0 ? 3 : 2) k_source(ZoneView z, const DMech *__restrict__ mech,
@@ -782,7 +782,8 @@ __global__ void __launch_bounds__(kTB) k_properties(ZoneView z, DParams P, const
     z.mul[q] = mu;
     z.cond[q] = lam;
     z.mach[q] = z.vel[q] / a;
-  }  if constexpr (PLANE) {
+  }
+  if constexpr (PLANE) {
     if (!dt_partial) return;
     double best = 1e+6;
     if (live && i >= 0 && i < z.mx && j >= 0 && j < z.my) {
