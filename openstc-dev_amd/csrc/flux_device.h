@@ -116,10 +116,12 @@ __device__ inline void recon_pv(const ZoneView &z, int recon, MechK m, int64_t p
 // AWENO.cu:151-206 WENO5 on the six characteristic values v[s] of the
 // stencil points s = 0..5 (i-2..i+3): v-(i+1/2) and v+(i+1/2).
 // The nonlinear weights a_k = c_k (1 + tau / (eps + b_k)^2) of each side
-// share one reciprocal of the product of their three denominators
-// (each denominator lies in [1e-12, 1e14] for characteristic variables in
-// density units, far from the double range), and the two normalisations
-// share one reciprocal of the product of the weight sums.
+// share one reciprocal of the product of their three denominators, and the two
+// normalisations share one reciprocal of the product of the weight sums.  A
+// denominator is about the fourth power of a jump of v (1e-12 at least): for
+// variables in density units it stays below 1e14, but rho k and rho omega jump
+// by 1e5 and 1e9 near a wall, denominators of 1e20 and 1e36, whose product is
+// inside the double range and far outside FP32's (weno5_wide).
 template <typename R>
 __device__ inline void weno5_vals(const R *v, R &vm, R &vp) {
   const R t12 = R(13.0 / 12), eps = R(1e-6);
@@ -150,6 +152,44 @@ __device__ inline void weno5_vals(const R *v, R &vm, R &vp) {
   const R is = rcp(sl * sr);
   vm = (al0 * u0 + al1 * u1 + al2 * u2) * (sr * is);
   vp = (ar0 * u1 + ar1 * u2 + ar2 * u3) * (sl * is);
+}
+
+// The same for rho k and rho omega in FP32, where weno5_vals turned NaN, by 0
+// times infinity, from jumps of 6e4 on, and the face fell back to first order
+// (three quarters of the faces of a channel's wall-normal sweep).  Here
+// r_k = (b_0 - b_2) / (eps + b_k) is formed for each candidate, limited to
+// 1e15 (what is left out is below FP32's resolution: such a candidate differs
+// from its neighbour by less than 3e-8 of the jump), and the weights are
+// normalised before they meet the candidates.
+template <typename R>
+__device__ inline void weno5_wide(const R *v, R &vm, R &vp) {
+  const R t12 = R(13.0 / 12), eps = R(1e-6), top = R(1e15);
+  const R o16 = R(1.0 / 16), f8 = R(5.0 / 8), f16 = R(5.0 / 16);
+  const R u0 = R(0.125) * (R(3) * v[0] - R(10) * v[1] + R(15) * v[2]);
+  const R u1 = R(0.125) * (-v[1] + R(6) * v[2] + R(3) * v[3]);
+  const R u2 = R(0.125) * (R(3) * v[2] + R(6) * v[3] - v[4]);
+  const R u3 = R(0.125) * (R(15) * v[3] - R(10) * v[4] + R(3) * v[5]);
+  // 13/12 of the squared second differences D_s = v[s-1] - 2 v[s] + v[s+1]
+  R e[6];
+#pragma unroll
+  for (int s = 1; s < 5; ++s) {
+    const R D = v[s - 1] + v[s + 1] - R(2) * v[s];
+    e[s] = t12 * D * D;
+  }
+  auto sq = [](R a) { return a * a; };
+  const R bl0 = e[1] + R(0.25) * sq(v[0] + R(3) * v[2] - R(4) * v[1]);
+  const R bl1 = e[2] + R(0.25) * sq(v[3] - v[1]);
+  const R bl2 = e[3] + R(0.25) * sq(R(3) * v[2] + v[4] - R(4) * v[3]);
+  const R br0 = e[2] + R(0.25) * sq(v[1] + R(3) * v[3] - R(4) * v[2]);
+  const R br1 = e[3] + R(0.25) * sq(v[4] - v[2]);
+  const R br2 = e[4] + R(0.25) * sq(R(3) * v[3] + v[5] - R(4) * v[4]);
+  const R tl = fabs(bl0 - bl2), tr = fabs(br0 - br2);
+  auto weight = [&](R c, R tau, R b) { return c + c * sq(fmin(tau * rcp(eps + b), top)); };
+  const R al0 = weight(o16, tl, bl0), al1 = weight(f8, tl, bl1), al2 = weight(f16, tl, bl2);
+  const R ar0 = weight(f16, tr, br0), ar1 = weight(f8, tr, br1), ar2 = weight(o16, tr, br2);
+  const R il = rcp(al0 + al1 + al2), ir = rcp(ar0 + ar1 + ar2);
+  vm = (al0 * il) * u0 + (al1 * il) * u1 + (al2 * il) * u2;
+  vp = (ar0 * ir) * u1 + (ar1 * ir) * u2 + (ar2 * ir) * u3;
 }
 
 // The same in first and second differences d, D of the stencil, for air: 2,211
@@ -555,7 +595,10 @@ __device__ inline void aweno_mix(const ZoneView &z, MechK m, int64_t p0, int64_t
       if (l < NS) c1[s] += E.a[l] * ql;
       v[s] = ql - E.y[l] * q[s][0];
     }
-    weno5_vals(v, wm[5 + l], wp[5 + l]);
+    if (sizeof(R) == 8 || l < NS)
+      weno5_vals(v, wm[5 + l], wp[5 + l]);
+    else
+      weno5_wide(v, wm[5 + l], wp[5 + l]);
   }
 #pragma unroll
   for (int s = 0; s < 6; ++s) {

@@ -111,3 +111,33 @@ def test_sst_plate_aweno(tmp_path):
     s.step(19)
     z.run(19)
     _compare_sst(s, z, 1e-9, "plate-aweno-20")
+
+
+@pytest.mark.parametrize("kind", ["channel", "plate"])
+def test_sst_fp32_fluxes(tmp_path, mech, kind):
+    """FP32 fluxes of the k and omega rows, whose values jump by 1e5 and 1e8
+    near the wall: the smoothness weights' products leave FP32's range there.
+    Bar: a face's value carries some 100 roundings of 2^-24 relative to the
+    largest terms of its row, and the right-hand side is the difference of two
+    faces.  In the momentum rows the largest term is the pressure on the face,
+    p |J grad xi|, which nearly cancels between two faces (the plate's rows
+    across the flow hold little else); elsewhere the differences of the terms
+    are within a factor of ten of the terms: 1e-4 of the row's largest entry.
+    With faces at first order, rows are off by 1e-3 to 1 of it."""
+    case, s, z = _c5(tmp_path, mech, recon=4) if kind == "channel" else _plate(tmp_path, nx=48, ny=32,
+                                                                              reconstruction=4)
+    if kind == "channel":
+        s.step_steady(2)
+    nv = s.get_int("n_var")
+    s.rhs()
+    a = s.download("dq").reshape(nv, -1)
+    s.set_flux_fp32(True)
+    s.rhs()
+    b = s.download("dq").reshape(nv, -1)
+    bar = 1e-4 * np.abs(a).max(axis=1)
+    jac = s.download("jac")
+    force = s.download("bv").reshape(6, -1)[4] * np.abs(jac * s.download("metric").reshape(9, -1)).max(axis=0)
+    bar[1:4] = 100 * 2.0 ** -24 * force.max()
+    err = np.abs(a - b).max(axis=1) / bar
+    print(kind, "FP32 fluxes, of the bar by row", ["%.1e" % e for e in err], flush=True)
+    assert np.isfinite(b).all() and err.max() < 1
