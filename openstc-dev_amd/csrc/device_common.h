@@ -118,8 +118,9 @@ constexpr double kMwAirD = 28.9647;
 // some 700 of the 980 vector loads of a 9-species AWENO face.  With the
 // branch-free forms, the mixture polynomial below and products with 1 / W_l
 // in place of quotients: 512x256 mixing layer 2.69 -> 1.71 ms per RK3 step,
-// 192x96x64 channel 12.5 -> 8.6 ms per pseudo-iteration; the 9-species AWENO
-// sweeps no longer use scratch memory.
+// 192x96x64 channel 12.5 -> 8.6 ms per pseudo-iteration; the laminar 9-species
+// AWENO sweeps no longer use scratch memory (with SST they use 76 to 148 B per
+// lane).
 typedef const __attribute__((address_space(4))) DMech *MechK;
 __device__ inline MechK mech_k(const DMech *m) { return (MechK)m; }
 
@@ -259,8 +260,10 @@ __device__ inline double d_species_gibbs(MechK m, int l, double t, double lt, do
 struct MixPoly {
   double a0, a1, a2, a3, a4, a5, ta, tb;
 
-  // the coefficients are loaded for two species at a time (fresh): loaded all
-  // at once they overflow the scalar registers into vector-register lanes
+  // fresh: the coefficients are loaded for two species at a time.  It orders
+  // the loads among themselves and not the arithmetic behind them, so in the
+  // sweeps most of a species' set still waits in vector-register lanes (1,036
+  // spilled scalar registers in the 9-species AWENO j-sweep)
   template <int NS>
   __device__ inline void build(MechK m, const double *w, double t) {
     a0 = a1 = a2 = a3 = a4 = a5 = 0;

@@ -197,7 +197,9 @@ __device__ inline void weno5_wide(const R *v, R &vm, R &vp) {
 // 256x128x128 air 5.27 -> 5.14 ms per step, 131x67x45 with FP32 fluxes 1.30 ->
 // 1.27 ms per 2 steps.  The mixture faces keep the form above: their sweeps
 // hold 500 registers and spilled more with this one, and the 9-species SST
-// parity case turned NaN after 18 pseudo-iterations.  The smoothness
+// parity case turned NaN after 18 pseudo-iterations, on faces that are finite
+// and the same to 1e-14 with both forms when this code is built for the CPU.
+// The smoothness
 // indicators are 13/12 D^2 + h^2 with h = d -+ D / 2 (four of the six share
 // their D), the candidates v[2] or v[3] plus combinations of the same d, D.
 // The nonlinear weights c_k (1 + tau / (eps + b_k)^2), multiplied by the three

@@ -39,8 +39,9 @@ __device__ inline double wave_sum(double v) {
 // are added to and the flow rows left alone.  One instantiation per method:
 // the Jacobian's registers would otherwise set the occupancy of the explicit
 // source too (1 wavefront per SIMD where it has 4).  131,072 cells of 9 species
-// and 19 reactions: 127 -> 41 us; 20,503 cells: 63 -> 33 us; with the Jacobian,
-// 1.18 M cells: 1.37 -> 0.55 ms (0.9 GB of it, the Jacobian's stores).
+// and 19 reactions: 127 -> 41 us; 20,503 cells: 63 -> 24 us; with the Jacobian,
+// 1.18 M cells: 1.37 -> 0.56 ms (0.9 GB of it, the Jacobian's stores), at 256
+// registers and 36 B of scratch per lane (180 B when the last species reacts).
 constexpr int kSrcTB = 128;
 constexpr int kMaxEpiReac = 24;  // reactions that the point-implicit paths accept (the batch parks their rates in LDS)
 
