@@ -42,6 +42,9 @@ __device__ inline double wave_sum(double v) {
 // and 19 reactions: 127 -> 41 us; 20,503 cells: 63 -> 24 us; with the Jacobian,
 // 1.18 M cells: 1.37 -> 0.56 ms (0.9 GB of it, the Jacobian's stores), at 256
 // registers and 36 B of scratch per lane (180 B when the last species reacts).
+// Methods 1 and 2 keep creation and destruction sums in LDS too, 40 KB per
+// workgroup with 9 species, which leaves 2 wavefronts per SIMD: the register
+// bound asks for no more than that.
 constexpr int kSrcTB = 128;
 constexpr int kMaxEpiReac = 24;  // reactions that the point-implicit paths accept (the batch parks their rates in LDS)
 
